@@ -21,6 +21,7 @@ ENTRY_POINTS = {
     "launch_h3_full_attention": 5,
     "launch_h3_full_attention_ws": 6,
     "launch_h3_vision_attention_72": 5,
+    "launch_h3_attention_planned": 6,
     "launch_h3_full_attention_bf16_prescale": 5,
     "launch_h3_full_attention_fp8": 8,
     "launch_h3_full_attention_fp8pv": 6,
@@ -107,18 +108,27 @@ def entry(name: str):
     return fn
 
 
+def _workspace_query(name: str, *sizes: int) -> int:
+    fn = _bound.get(name)
+    if fn is None:
+        fn = getattr(library(), name)
+        fn.restype = ctypes.c_int64
+        fn.argtypes = [ctypes.c_int64] * len(sizes)
+        _bound[name] = fn
+    n = int(fn(*sizes))
+    if n < 0:
+        raise LaunchError(name, 100)
+    return n
+
+
 def attention_workspace_bytes(B: int, H: int, Sq: int, Sk: int) -> int:
     """h3_full_attention_workspace_bytes on the current device (0: no split)."""
-    fn = _bound.get("h3_full_attention_workspace_bytes")
-    if fn is None:
-        fn = library().h3_full_attention_workspace_bytes
-        fn.restype = ctypes.c_int64
-        fn.argtypes = [ctypes.c_int64] * 4
-        _bound["h3_full_attention_workspace_bytes"] = fn
-    n = int(fn(B, H, Sq, Sk))
-    if n < 0:
-        raise LaunchError("h3_full_attention_workspace_bytes", 100)
-    return n
+    return _workspace_query("h3_full_attention_workspace_bytes", B, H, Sq, Sk)
+
+
+def attention_planned_workspace_bytes(B: int, H: int, Sq: int, Sk: int, head_dim: int) -> int:
+    """h3_attention_planned_workspace_bytes on the current device (0: none used)."""
+    return _workspace_query("h3_attention_planned_workspace_bytes", B, H, Sq, Sk, head_dim)
 
 
 def _error_string(status: int) -> str:

@@ -24,11 +24,11 @@
 //     and denominator in the workspace and a merge kernel combines them (the
 //     same algebra as the online rescale).
 //
-// attention16_kernel (D = 128 on the buffer path: the configurations) runs on
-// v_mfma_f32_16x16x32_bf16 and keeps one reference maximum per unit (its
-// layout and numerics are described above it). attention_fwd_kernel runs on
-// v_mfma_f32_32x32x16_bf16 with the exact online rescale and serves D = 72
-// and K/V views outside the buffer path:
+// attention16_kernel (the buffer path: the configurations and the vision
+// tower) runs on v_mfma_f32_16x16x32_bf16 and keeps one reference maximum per
+// unit (its layout and numerics are described above it). attention_fwd_kernel
+// runs on v_mfma_f32_32x32x16_bf16 with the exact online rescale and serves
+// K/V views outside the buffer path and D = 72 launches that leave CUs idle:
 //
 // MFMA formulation (v_mfma_f32_32x32x16_bf16; A row = lane % 32, B column =
 // lane % 32, accumulator register i of lane l holds row 8*(i/4) + 4*(l/32) + i%4)
@@ -104,7 +104,7 @@ struct AttnArgs {
     // n_full + u, (p, u) = (lp / n_tail, lp % n_tail) for lp the XCD-remapped
     // j: key tiles [p T / split, (p + 1) T / split) of the unit's T tiles.
     int n_full, n_tail, split;
-    float *ws;                            // the partials (layout at kWsSlotAcc)
+    float *ws;                            // the partials (layout at ws_slot_acc)
     // SMALL kernels: workgroups [0, n_big) run 256-query units and workgroups
     // [n_big, n_big + n_small) 192-query units, each range XCD-remapped on its
     // own, so the 192-query units make up the last round. A head (b H + h)
@@ -126,11 +126,11 @@ struct SmallUnit {
 __device__ __forceinline__ SmallUnit small_plan_unit(const AttnArgs &a, int x);
 
 // Workspace of the SPLIT kernels, per piece slot (u split + p): the
-// unnormalised O as [256 queries][128 dims] floats, then, after all slots'
+// unnormalised O as [256 queries][D dims] floats, then, after all slots'
 // O, the reference maximum and the denominator as [256 queries][2] floats.
-constexpr int kWsSlotAcc = kBM * kD;
+__host__ __device__ constexpr int ws_slot_acc(int dim) { return kBM * dim; }
 constexpr int kWsSlotMl = kBM * 2;
-constexpr int64_t kWsSlotBytes = static_cast<int64_t>(kWsSlotAcc + kWsSlotMl) * 4;
+constexpr int64_t ws_slot_bytes(int dim) { return static_cast<int64_t>(ws_slot_acc(dim) + kWsSlotMl) * 4; }
 constexpr int kMaxSplit = 8;
 
 // The dword-3 word of a raw buffer descriptor on gfx9 (CDNA): no format
@@ -577,7 +577,7 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
 
 // ============================================================ attention16_kernel
 //
-// The D = 128 kernel on the buffer path, on v_mfma_f32_16x16x32_bf16: under
+// The kernel of the buffer path, on v_mfma_f32_16x16x32_bf16: under
 // power the part sustains about 14% more flops with this product than with
 // 32x32x16 (launch_h3_calibration_mfma_16x16x32).
 //
@@ -621,6 +621,22 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
 
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
+// The 32-dim k-steps of Q K^T and the 16-dim blocks of O^T: 4 and 8 at
+// D = 128, 3 and 5 at D = 72 (dims 72..95 and 72..79 are padding).
+template <int DIM>
+constexpr int k_steps16() { return (DIM + 31) / 32; }
+template <int DIM>
+constexpr int dim_blocks16() { return (DIM + 15) / 16; }
+
+// The byte offset of chunk `chunk` (8 dims) of key row `row` in a head's rows;
+// chunks past the head dim lie past any descriptor's range (which, with every
+// tile offset, stays below 2^30) and read as zero.
+template <int DIM>
+__device__ __forceinline__ int chunk_offset(int row, int chunk, int64_t stride) {
+    const int at = (row * static_cast<int>(stride) + 8 * chunk) * 2;
+    return DIM == kD || chunk < DIM / 8 ? at : kBeyondRange;
+}
+
 // V tile swizzle of this kernel: chunk c of row r at slot c ^ 2 (r & 7), so
 // the 8 consecutive rows x 2 chunks one half-wave's ds_read_b64_tr_b16 reads
 // land on 16 distinct slots.
@@ -640,19 +656,19 @@ __device__ __forceinline__ float fold_groups_max(float x) {
 // S^T of one 64-key tile for NQB 16-query blocks. kidx: this lane's K operand
 // element for k-step 0 (row 16 kb + l % 16 of the tile, chunk 4 ks + l / 16;
 // k-step ks reads kidx ^ 32 ks). Each K operand feeds every query block.
-template <int NQB>
-__device__ __forceinline__ void qk_tile16(const bf16_t *kt, const bf16x8_t (&qreg)[NQB][4], int kidx,
-                                          f32x4_t (&s)[NQB][4]) {
+template <int NQB, int KS, int KB>
+__device__ __forceinline__ void qk_tile16(const bf16_t *kt, const bf16x8_t (&qreg)[NQB][KS], int kidx,
+                                          f32x4_t (&s)[NQB][KB]) {
 #pragma unroll
     for (int qb = 0; qb < NQB; ++qb)
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb)
+        for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
             for (int i = 0; i < 4; ++i) s[qb][kb][i] = 0.0f;
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks)
+    for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb) {
+        for (int kb = 0; kb < KB; ++kb) {
             const bf16x8_t kop = as_bf16x8(*reinterpret_cast<const uint4 *>(kt + 16 * kb * kRow + (kidx ^ (32 * ks))));
 #pragma unroll
             for (int qb = 0; qb < NQB; ++qb)
@@ -663,7 +679,7 @@ __device__ __forceinline__ void qk_tile16(const bf16_t *kt, const bf16x8_t (&qre
     // deeper V^T window, lose).
     __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
 #pragma unroll
-    for (int i = 0; i < 12; ++i) {
+    for (int i = 0; i < KB * KS - 4; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, NQB, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
     }
@@ -675,15 +691,15 @@ __device__ __forceinline__ void qk_tile16(const bf16_t *kt, const bf16x8_t (&qre
 // vidx: this lane's V^T operand address for dim block 0 of the lower 4 keys
 // (row 4 (l / 16) + (l % 16) / 4, dims 4 (l % 4) of the block; block db reads
 // vidx ^ 16 db, the upper 4 keys 16 rows further, half h 32 rows further).
-template <bool MASK, int NQB>
-__device__ __forceinline__ void pv_tile16(const bf16_t *vt, int vidx, const f32x4_t (&s)[NQB][4], const float (&m)[NQB],
-                                          f32x4_t (&l)[NQB], float c, int valid, int g, f32x4_t (&acc)[NQB][8]) {
-    bf16x8_t pop[NQB][2];
+template <bool MASK, int NQB, int DB, int KB>
+__device__ __forceinline__ void pv_tile16(const bf16_t *vt, int vidx, const f32x4_t (&s)[NQB][KB], const float (&m)[NQB],
+                                          f32x4_t (&l)[NQB], float c, int valid, int g, f32x4_t (&acc)[NQB][DB]) {
+    bf16x8_t pop[NQB][KB / 2];
 #pragma unroll
     for (int qb = 0; qb < NQB; ++qb) {
-        float p[4][4];
+        float p[KB][4];
 #pragma unroll
-        for (int kb = 0; kb < 4; ++kb)
+        for (int kb = 0; kb < KB; ++kb)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 float e = __builtin_amdgcn_exp2f(__builtin_fmaf(s[qb][kb][i], c, -m[qb]));
@@ -693,7 +709,7 @@ __device__ __forceinline__ void pv_tile16(const bf16_t *vt, int vidx, const f32x
                 p[kb][i] = e;
             }
 #pragma unroll
-        for (int h = 0; h < 2; ++h) {
+        for (int h = 0; h < KB / 2; ++h) {
             uint4 packed;
             packed.x = pack2(p[2 * h][0], p[2 * h][1]);
             packed.y = pack2(p[2 * h][2], p[2 * h][3]);
@@ -703,23 +719,29 @@ __device__ __forceinline__ void pv_tile16(const bf16_t *vt, int vidx, const f32x
         }
     }
     // The denominator on the matrix core: ones x P^T adds the 32 keys of each
-    // half to every row of l (each lane then holds its query's whole sum).
-    {
+    // half to every row of l (each lane then holds its query's whole sum). At
+    // D = 72 dim 72 of V is taken as ones, and the sum falls out of P V.
+    if constexpr (DB == dim_blocks16<kD>()) {
         const bf16x8_t ones = as_bf16x8(make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+        for (int h = 0; h < KB / 2; ++h)
 #pragma unroll
             for (int qb = 0; qb < NQB; ++qb) l[qb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ones, pop[qb][h], l[qb], 0, 0, 0);
     }
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+    for (int h = 0; h < KB / 2; ++h)
 #pragma unroll
-        for (int db = 0; db < 8; ++db) {
+        for (int db = 0; db < DB; ++db) {
             const bf16_t *vp = vt + 32 * h * kRow + (vidx ^ (16 * db));
             const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t *)(vp));
             const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t *)(vp + 16 * kRow));
             const uint2 lo2 = __builtin_bit_cast(uint2, lo), hi2 = __builtin_bit_cast(uint2, hi);
-            const bf16x8_t vop = as_bf16x8(make_uint4(lo2.x, lo2.y, hi2.x, hi2.y));
+            uint4 vw = make_uint4(lo2.x, lo2.y, hi2.x, hi2.y);
+            if (DB != dim_blocks16<kD>() && db == DB - 1) {  // dim 72's row: ones over its zeros
+                const uint32_t one = (threadIdx.x & 15) == 8 ? 0x3f803f80u : 0u;
+                vw = make_uint4(vw.x | one, vw.y | one, vw.z | one, vw.w | one);
+            }
+            const bf16x8_t vop = as_bf16x8(vw);
 #pragma unroll
             for (int qb = 0; qb < NQB; ++qb)
                 acc[qb][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop, pop[qb][h], acc[qb][db], 0, 0, 0);
@@ -727,7 +749,7 @@ __device__ __forceinline__ void pv_tile16(const bf16_t *vt, int vidx, const f32x
     // Rolling window of V^T operand reads (two per operand), two operands ahead.
     __builtin_amdgcn_sched_group_barrier(0x100, 4, 0);
 #pragma unroll
-    for (int i = 0; i < 14; ++i) {
+    for (int i = 0; i < KB / 2 * DB - 2; ++i) {
         __builtin_amdgcn_sched_group_barrier(0x008, NQB, 0);
         __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
     }
@@ -738,10 +760,10 @@ __device__ __forceinline__ void pv_tile16(const bf16_t *vt, int vidx, const f32x
 // raises the running maximum m of some query, O and the denominator scaled by
 // exp2(m_old - m_new) first (the reference's order). From m = -inf, l = 0,
 // O = 0 it sets the reference maximum of the first tile.
-template <bool MASK, bool NEG, int NQB>
+template <bool MASK, bool NEG, int NQB, int KS, int DB>
 __device__ __forceinline__ void exact_tile16(const bf16_t *kt, const bf16_t *vt, int valid,
-                                             const bf16x8_t (&qreg)[NQB][4], int kidx, int vidx, int g, float c,
-                                             float (&m)[NQB], f32x4_t (&l)[NQB], f32x4_t (&acc)[NQB][8]) {
+                                             const bf16x8_t (&qreg)[NQB][KS], int kidx, int vidx, int g, float c,
+                                             float (&m)[NQB], f32x4_t (&l)[NQB], f32x4_t (&acc)[NQB][DB]) {
     static_assert(NQB == 1 || NQB == 2, "one or two query blocks per wave");
     f32x4_t s[NQB][4];
     qk_tile16(kt, qreg, kidx, s);
@@ -772,7 +794,7 @@ __device__ __forceinline__ void exact_tile16(const bf16_t *kt, const bf16_t *vt,
             l[0] *= a0;
             l[1] *= a1;
 #pragma unroll
-            for (int db = 0; db < 8; ++db)
+            for (int db = 0; db < DB; ++db)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     acc[0][db][i] *= a0;
@@ -787,7 +809,7 @@ __device__ __forceinline__ void exact_tile16(const bf16_t *kt, const bf16_t *vt,
             m[0] = n0;
             l[0] *= a0;
 #pragma unroll
-            for (int db = 0; db < 8; ++db)
+            for (int db = 0; db < DB; ++db)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) acc[0][db][i] *= a0;
         }
@@ -795,32 +817,90 @@ __device__ __forceinline__ void exact_tile16(const bf16_t *kt, const bf16_t *vt,
     pv_tile16<MASK>(vt, vidx, s, m, l, c, valid, g, acc);
 }
 
+// exact_tile16 with a query block's O rescaled only when one of its own
+// queries' maxima grows, and the cross-lane fold of the maxima run only then:
+// some lane's own maximum exceeds the running one exactly when the folded one
+// does.
+template <bool MASK, bool NEG, int KB, int NQB, int KS, int DB>
+__device__ __forceinline__ void running_tile16(const bf16_t *kt, const bf16_t *vt, int valid,
+                                               const bf16x8_t (&qreg)[NQB][KS], int kidx, int vidx, int g, float c,
+                                               float (&m)[NQB], f32x4_t (&l)[NQB], f32x4_t (&acc)[NQB][DB]) {
+    f32x4_t s[NQB][KB];
+    qk_tile16(kt, qreg, kidx, s);
+    float mx[NQB];
+#pragma unroll
+    for (int qb = 0; qb < NQB; ++qb) {
+        if constexpr (MASK) {
+#pragma unroll
+            for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    if (16 * kb + 4 * g + i >= valid) s[qb][kb][i] = NEG ? INFINITY : -INFINITY;
+        }
+        mx[qb] = s[qb][0][0];
+#pragma unroll
+        for (int kb = 0; kb < KB; ++kb)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) mx[qb] = NEG ? fminf(mx[qb], s[qb][kb][i]) : fmaxf(mx[qb], s[qb][kb][i]);
+    }
+#pragma unroll
+    for (int qb = 0; qb < NQB; ++qb) {
+        if (__builtin_amdgcn_ballot_w64(mx[qb] * c > m[qb])) {
+            const float mt = fold_groups_max<NEG>(mx[qb]) * c;
+            const float n = mt > m[qb] ? mt : m[qb];
+            const float al = __builtin_amdgcn_exp2f(m[qb] - n);
+            m[qb] = n;
+            if constexpr (DB == dim_blocks16<kD>()) l[qb] *= al;
+#pragma unroll
+            for (int db = 0; db < DB; ++db)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) acc[qb][db][i] *= al;
+        }
+    }
+    pv_tile16<MASK>(vt, vidx, s, m, l, c, valid, g, acc);
+}
+
 // A tile against the fixed reference maximum m.
-template <bool MASK, int NQB>
+template <bool MASK, int KB, int NQB, int KS, int DB>
 __device__ __forceinline__ void ref_tile16(const bf16_t *kt, const bf16_t *vt, int valid,
-                                           const bf16x8_t (&qreg)[NQB][4], int kidx, int vidx, int g, float c,
-                                           const float (&m)[NQB], f32x4_t (&l)[NQB], f32x4_t (&acc)[NQB][8]) {
-    f32x4_t s[NQB][4];
+                                           const bf16x8_t (&qreg)[NQB][KS], int kidx, int vidx, int g, float c,
+                                           const float (&m)[NQB], f32x4_t (&l)[NQB], f32x4_t (&acc)[NQB][DB]) {
+    f32x4_t s[NQB][KB];
     qk_tile16(kt, qreg, kidx, s);
     pv_tile16<MASK>(vt, vidx, s, m, l, c, valid, g, acc);
 }
 
-// A query's denominator: every row of its l accumulator holds the whole sum.
-__device__ __forceinline__ float den_total(const f32x4_t &l) { return l[0]; }
+// A query's denominator: every row of its l accumulator holds the whole sum;
+// at D = 72 it is O^T's row 72, register 0 of dim block 4 in lane group 2.
+template <int DB>
+__device__ __forceinline__ float den_total(const f32x4_t &l, const f32x4_t (&acc)[DB], int l16) {
+    if constexpr (DB == dim_blocks16<kD>())
+        return l[0];
+    else
+        return __shfl(acc[4][0], 32 + l16, 64);
+}
 
 // The Q^T operands of query block qb (k-step ks: dims 32 ks + 8 g .. +8 of
 // query q_first + 16 qb + l16, clamped to the last query), prescaled to
 // bf16(fp32(c) * fp32(q)) for the prescale numerics (tools/h3_attention.py:88).
+template <int KS>
 __device__ __forceinline__ void load_q16(const AttnArgs &a, const bf16_t *qbase, int q_first, int qb, int l16, int g,
-                                         bf16x8_t (&qr)[4]) {
+                                         bf16x8_t (&qr)[KS]) {
     int query = q_first + 16 * qb + l16;
     query = query < a.Sq ? query : a.Sq - 1;
     const bf16_t *qrow = qbase + static_cast<int64_t>(query) * a.qs[2];
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) qr[ks] = as_bf16x8(*reinterpret_cast<const uint4 *>(qrow + 32 * ks + 8 * g));
+    for (int ks = 0; ks < KS; ++ks) {
+        if (KS == k_steps16<kD>() || ks < 2) {
+            qr[ks] = as_bf16x8(*reinterpret_cast<const uint4 *>(qrow + 32 * ks + 8 * g));
+        } else {  // D = 72: dims 64..71 in group 0, zeros past them
+            const uint4 u = *reinterpret_cast<const uint4 *>(qrow + 32 * ks);
+            qr[ks] = as_bf16x8(g == 0 ? u : make_uint4(0u, 0u, 0u, 0u));
+        }
+    }
     if (a.prescale) {
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
+        for (int ks = 0; ks < KS; ++ks) {
             const uint4 u = __builtin_bit_cast(uint4, qr[ks]);
             const uint32_t w[4] = {u.x, u.y, u.z, u.w};
             uint32_t o[4];
@@ -833,7 +913,13 @@ __device__ __forceinline__ void load_q16(const AttnArgs &a, const bf16_t *qbase,
 
 // SPLIT: the key-split launch (see AttnArgs); a piece leaves its unnormalised
 // O, reference maximum and denominator in the workspace for the merge.
-template <bool NEG, bool SPLIT>
+// DIM: the head dim, 128 or 72. At 72 the tiles keep the 128-dim row layout
+// (chunks past the head dim are zeros), 3 k-steps and 5 dim blocks hold the 72
+// dims, and dim 72's row of O^T is the denominator: 44 products per tile and
+// wave. It keeps the running maximum: against a fixed one its error against
+// float64 was 2-5% larger than the 32x32x16 kernel's it replaces, with it 1-3%
+// smaller (over S = 256 .. 16,384, N(0, 1) and 1% of key rows x8).
+template <bool NEG, bool SPLIT, int DIM>
 __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWaves / 4, kWaves / 4))) void attention16_kernel(AttnArgs a) {
     __shared__ __attribute__((aligned(1024))) bf16_t lds_k0[kTileElems];
     __shared__ __attribute__((aligned(1024))) bf16_t lds_k1[kTileElems];
@@ -867,7 +953,8 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
     // Q^T operands: query block qb, k-step ks holds dims 32 ks + 8 g .. +8 of
     // query 16 qb + l16 of this wave's 32.
     const int q_first = qbk * kBM + wave * 32;
-    bf16x8_t qreg[2][4];
+    constexpr int KS = k_steps16<DIM>(), DB = dim_blocks16<DIM>();
+    bf16x8_t qreg[2][KS];
     load_q16(a, qbase, q_first, 0, l16, g, qreg[0]);
     load_q16(a, qbase, q_first, 1, l16, g, qreg[1]);
 
@@ -880,8 +967,8 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
 #pragma unroll
     for (int r = 0; r < kLoadRows; ++r) {
         const int row = tile_row(r);
-        kvoff[r] = (row * static_cast<int>(a.ks[2]) + 8 * (static_cast<int>(threadIdx.x & 15) ^ swz_k(row))) * 2;
-        vvoff[r] = (row * static_cast<int>(a.vs[2]) + 8 * (static_cast<int>(threadIdx.x & 15) ^ swz_v16(row))) * 2;
+        kvoff[r] = chunk_offset<DIM>(row, static_cast<int>(threadIdx.x & 15) ^ swz_k(row), a.ks[2]);
+        vvoff[r] = chunk_offset<DIM>(row, static_cast<int>(threadIdx.x & 15) ^ swz_v16(row), a.vs[2]);
     }
     const int kidx = l16 * kRow + 8 * (g ^ l16);
     const int vrow = 4 * g + (l16 >> 2);
@@ -903,7 +990,7 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
     }
     const int valid_last = a.Sk - full * kBN;
 
-    f32x4_t acc[2][8];
+    f32x4_t acc[2][DB];
     float m[2];
     f32x4_t l[2];
     // One pass over the unit's tiles for the query blocks of qq (one or two;
@@ -911,14 +998,14 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
     // first tile exact (it sets the reference maxima), the rest against them
     // (EXACT: all with the online rescale).
     auto pass = [&](auto exact_tag, const auto &qq, auto &mm, auto &ll, auto &aa) __attribute__((always_inline)) {
-        constexpr bool EXACT = decltype(exact_tag)::value;
+        constexpr bool EXACT = DIM != kD || decltype(exact_tag)::value;
         constexpr int NQ = sizeof(mm) / sizeof(float);
 #pragma unroll
         for (int qb = 0; qb < NQ; ++qb) {
             mm[qb] = -INFINITY;
             ll[qb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-            for (int db = 0; db < 8; ++db)
+            for (int db = 0; db < DB; ++db)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) aa[qb][db][i] = 0.0f;
         }
@@ -933,9 +1020,9 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
             dma_tile(krs, kvoff, (tile + 1) * kstep, kn);
             dma_tile(vrs, vvoff, (tile + 1) * vstep, vn);
             if constexpr (EXACT || decltype(first_tag)::value)
-                exact_tile16<false, NEG>(kc, vc, kBN, qq, kidx, vidx, g, c, mm, ll, aa);
+                running_tile16<false, NEG, 4>(kc, vc, kBN, qq, kidx, vidx, g, c, mm, ll, aa);
             else
-                ref_tile16<false>(kc, vc, kBN, qq, kidx, vidx, g, c, mm, ll, aa);
+                ref_tile16<false, 4>(kc, vc, kBN, qq, kidx, vidx, g, c, mm, ll, aa);
             asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
             __syncthreads();
         };
@@ -952,12 +1039,12 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
                 const bf16_t *kc = odd ? lds_k1 : lds_k0;
                 const bf16_t *vc = odd ? lds_v1 : lds_v0;
                 if constexpr (EXACT)
-                    exact_tile16<true, NEG>(kc, vc, valid_last, qq, kidx, vidx, g, c, mm, ll, aa);
+                    running_tile16<true, NEG, 4>(kc, vc, valid_last, qq, kidx, vidx, g, c, mm, ll, aa);
                 else
-                    ref_tile16<true>(kc, vc, valid_last, qq, kidx, vidx, g, c, mm, ll, aa);
+                    ref_tile16<true, 4>(kc, vc, valid_last, qq, kidx, vidx, g, c, mm, ll, aa);
             }
         } else if (partial) {  // the partial tile is the only one
-            exact_tile16<true, NEG>(lds_k0, lds_v0, valid_last, qq, kidx, vidx, g, c, mm, ll, aa);
+            running_tile16<true, NEG, 4>(lds_k0, lds_v0, valid_last, qq, kidx, vidx, g, c, mm, ll, aa);
         }
     };
     pass(std::false_type{}, qreg, m, l, acc);
@@ -969,14 +1056,14 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
     // its last LDS read of the pass before the barrier.
     float lt[2];
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb) lt[qb] = den_total(l[qb]);
+    for (int qb = 0; qb < 2; ++qb) lt[qb] = den_total(l[qb], acc[qb], l16);
     const float limit = piece >= 0 ? __FLT_MAX__ / kMaxSplit : INFINITY;
     // x < limit is false for NaN, so NaN counts as overflow too.
     bool finite = lt[0] < limit && lt[1] < limit;
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
-        for (int db = 0; db < 8; ++db)
+        for (int db = 0; db < DB; ++db)
 #pragma unroll
             for (int i = 0; i < 4; ++i) finite = finite && fabsf(acc[qb][db][i]) < limit;
     const bool wave_bad = __builtin_amdgcn_ballot_w64(!finite) != 0;
@@ -991,11 +1078,11 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
         // (the kernel's register peak otherwise).
         auto redo = [&](auto qb_tag) __attribute__((always_inline)) {
             constexpr int qb = decltype(qb_tag)::value;
-            bf16x8_t q1[1][4];
+            bf16x8_t q1[1][KS];
             load_q16(a, qbase, q_first, qb, l16, g, q1[0]);
             pass(std::true_type{}, q1, *reinterpret_cast<float(*)[1]>(&m[qb]), *reinterpret_cast<f32x4_t(*)[1]>(&l[qb]),
-                 *reinterpret_cast<f32x4_t(*)[1][8]>(&acc[qb]));
-            lt[qb] = den_total(l[qb]);
+                 *reinterpret_cast<f32x4_t(*)[1][DB]>(&acc[qb]));
+            lt[qb] = den_total(l[qb], acc[qb], l16);
         };
         redo(std::integral_constant<int, 0>{});
         __syncthreads();  // every wave past its last LDS read
@@ -1004,15 +1091,16 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
     if constexpr (SPLIT) {
         if (piece >= 0) {  // a piece: O, m and l of its 256 queries go to the workspace
             const int64_t slot = static_cast<int64_t>(logical - a.n_full) * a.split + piece;
-            float *pa = a.ws + slot * kWsSlotAcc;
-            float *pm = a.ws + static_cast<int64_t>(a.n_tail) * a.split * kWsSlotAcc + slot * kWsSlotMl;
+            float *pa = a.ws + slot * ws_slot_acc(DIM);
+            float *pm = a.ws + static_cast<int64_t>(a.n_tail) * a.split * ws_slot_acc(DIM) + slot * kWsSlotMl;
 #pragma unroll
             for (int qb = 0; qb < 2; ++qb) {
                 const int r = wave * 32 + 16 * qb + l16;
 #pragma unroll
-                for (int db = 0; db < 8; ++db)
-                    *reinterpret_cast<float4 *>(pa + r * kD + 16 * db + 4 * g) =
-                        float4{acc[qb][db][0], acc[qb][db][1], acc[qb][db][2], acc[qb][db][3]};
+                for (int db = 0; db < DB; ++db)
+                    if (DIM % 16 == 0 || 16 * db + 4 * g < DIM)
+                        *reinterpret_cast<float4 *>(pa + r * DIM + 16 * db + 4 * g) =
+                            float4{acc[qb][db][0], acc[qb][db][1], acc[qb][db][2], acc[qb][db][3]};
                 if (g == 0) *reinterpret_cast<float2 *>(pm + 2 * r) = float2{m[qb], lt[qb]};
             }
             return;
@@ -1027,11 +1115,11 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
         const float inv = __fdiv_rn(1.0f, lt[qb]);
         bf16_t *orow = obase + static_cast<int64_t>(query) * a.os[2];
 #pragma unroll
-        for (int db = 0; db < 8; ++db) {
+        for (int db = 0; db < DB; ++db) {
             uint2 w;
             w.x = pack2(acc[qb][db][0] * inv, acc[qb][db][1] * inv);
             w.y = pack2(acc[qb][db][2] * inv, acc[qb][db][3] * inv);
-            *reinterpret_cast<uint2 *>(orow + 16 * db + 4 * g) = w;
+            if (DIM % 16 == 0 || 16 * db + 4 * g < DIM) *reinterpret_cast<uint2 *>(orow + 16 * db + 4 * g) = w;
         }
     }
 }
@@ -1125,7 +1213,7 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
                 if constexpr (EXACT || decltype(first_tag)::value)
                     exact_tile16<false, NEG>(kc, vc, kBN, qq, kidx, vidx, g, c, mm, ll, aa);
                 else
-                    ref_tile16<false>(kc, vc, kBN, qq, kidx, vidx, g, c, mm, ll, aa);
+                    ref_tile16<false, 4>(kc, vc, kBN, qq, kidx, vidx, g, c, mm, ll, aa);
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
                 __syncthreads();
             };
@@ -1144,7 +1232,7 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
                     if constexpr (EXACT)
                         exact_tile16<true, NEG>(kc, vc, valid_last, qq, kidx, vidx, g, c, mm, ll, aa);
                     else
-                        ref_tile16<true>(kc, vc, valid_last, qq, kidx, vidx, g, c, mm, ll, aa);
+                        ref_tile16<true, 4>(kc, vc, valid_last, qq, kidx, vidx, g, c, mm, ll, aa);
                 }
             } else if (partial) {  // the partial tile is the only one
                 exact_tile16<true, NEG>(lds_k0, lds_v0, valid_last, qq, kidx, vidx, g, c, mm, ll, aa);
@@ -1155,7 +1243,7 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
         // maximum (as attention16_kernel does).
         float lt[NQB];
 #pragma unroll
-        for (int qb = 0; qb < NQB; ++qb) lt[qb] = den_total(l[qb]);
+        for (int qb = 0; qb < NQB; ++qb) lt[qb] = den_total(l[qb], acc[qb], l16);
         constexpr float limit = INFINITY;
         // x < limit is false for NaN, so NaN counts as overflow too.
         bool finite = true;
@@ -1183,7 +1271,7 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
                 load_q16(a, qbase, q_first, qb, l16, g, q1[0]);
                 pass(std::true_type{}, q1, *reinterpret_cast<float(*)[1]>(&m[qb]),
                      *reinterpret_cast<f32x4_t(*)[1]>(&l[qb]), *reinterpret_cast<f32x4_t(*)[1][8]>(&acc[qb]));
-                lt[qb] = den_total(l[qb]);
+                lt[qb] = den_total(l[qb], acc[qb], l16);
             };
             redo(std::integral_constant<int, 0>{});
             __syncthreads();  // every wave past its last LDS read
@@ -1212,11 +1300,225 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
         run(std::integral_constant<int, 2>{});
 }
 
+// The kernel of launches with few units: 32 QW queries per workgroup (QW = 2
+// or 4), the keys of every 128-key tile split over its waves. Wave w takes the
+// 32 queries w % QW of the unit against key group w / QW of each tile (8 / QW
+// groups of 16 QW keys), so a wave's products keep the operand reuse of
+// attention16_kernel (each K and V operand feeds two query blocks) while the
+// launch has 8 / QW times as many workgroups and each half as many tile steps.
+// Each wave has its own reference maximum (its share of the first tile; D = 72:
+// the running maximum), and the key groups' O, maxima and denominators meet in
+// LDS, over the tile buffers, with the merge kernel's algebra: no workspace, no
+// second launch. What bounds it is latency: a tile step takes 1.1 us (QW = 2) or
+// 1.58 us (QW = 4), the rate of attention16_kernel's steps for its share of the
+// chip, after 7 us of launch, first loads and merge. 14 heads, S = 1024: 14.3
+// against 29.2 us (256-query units split in 2 over workgroups, and the merge
+// launch); S = 256: 9.1 against 14.1 us; S = 2048: 33.1 against 41.8 us; 16 heads
+// of 72, S = 1000: 13.8 against 25.1 us.
+constexpr int kShortBN = 128;  // keys per tile
+constexpr int kShortLoads = kShortBN * 16 / kThreadsWG;
+
+template <bool NEG, int DIM, int QW>
+__global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(2, 2))) void attention16_short_kernel(AttnArgs a) {
+    constexpr int KS = k_steps16<DIM>(), DB = dim_blocks16<DIM>();
+    constexpr int kQueries = 32 * QW;         // per workgroup
+    constexpr int kGroups = kWaves / QW;      // key groups
+    constexpr int kKeys = kShortBN / kGroups; // a wave's keys of a tile
+    constexpr int KB = kKeys / 16;
+    constexpr int kElems = kShortBN * kRow;
+    __shared__ __attribute__((aligned(1024))) bf16_t lds_k0[kElems];
+    __shared__ __attribute__((aligned(1024))) bf16_t lds_k1[kElems];
+    __shared__ __attribute__((aligned(1024))) bf16_t lds_v0[kElems];
+    __shared__ __attribute__((aligned(1024))) bf16_t lds_v1[kElems];
+    __shared__ float2 state[kGroups][kQueries];  // each key group's (maximum, denominator) per query
+    __shared__ int wave_overflow[kWaves];
+    static_assert(64 * kD * 4 == kElems * 2 && kGroups * kQueries == 256, "64 queries' O fill one tile buffer");
+
+    const int logical = xcd_remap(blockIdx.x, a.B * a.H * a.qblocks);
+    const int qbk = logical % a.qblocks, bh = logical / a.qblocks;
+    const int b = bh / a.H, h = bh % a.H;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int l16 = lane & 15, g = lane >> 4;
+    const int qw = wave % QW, kw = wave / QW;
+    const bf16_t *qbase = a.q + b * a.qs[0] + h * a.qs[1];
+    const bf16_t *kbase = a.k + b * a.ks[0] + h * a.ks[1];
+    const bf16_t *vbase = a.v + b * a.vs[0] + h * a.vs[1];
+    bf16_t *obase = a.o + b * a.os[0] + h * a.os[1];
+
+    const __amdgpu_buffer_rsrc_t krs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(kbase), static_cast<short>(0), a.k_bytes, kBufferWord3);
+    const __amdgpu_buffer_rsrc_t vrs =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t *>(vbase), static_cast<short>(0), a.v_bytes, kBufferWord3);
+    // Load i of wave w fills tile rows 4 (kShortLoads w + i) .. +3 (as tile_row).
+    int kvoff[kShortLoads], vvoff[kShortLoads];
+    const int kstep = static_cast<int>(a.ks[2]) * 2 * kShortBN, vstep = static_cast<int>(a.vs[2]) * 2 * kShortBN;
+#pragma unroll
+    for (int i = 0; i < kShortLoads; ++i) {
+        const int row = 4 * (kShortLoads * wave + i) + lane / 16;
+        kvoff[i] = chunk_offset<DIM>(row, l16 ^ swz_k(row), a.ks[2]);
+        vvoff[i] = chunk_offset<DIM>(row, l16 ^ swz_v16(row), a.vs[2]);
+    }
+    auto load_tiles = [&](int tile, bf16_t *kn, bf16_t *vn) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < kShortLoads; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                krs, (__attribute__((address_space(3))) void *)(kn + 4 * kRow * (kShortLoads * wave + i)), 16,
+                kvoff[i], tile * kstep, 0, 0);
+#pragma unroll
+        for (int i = 0; i < kShortLoads; ++i)
+            __builtin_amdgcn_raw_ptr_buffer_load_lds(
+                vrs, (__attribute__((address_space(3))) void *)(vn + 4 * kRow * (kShortLoads * wave + i)), 16,
+                vvoff[i], tile * vstep, 0, 0);
+    };
+    load_tiles(0, lds_k0, lds_v0);
+    const int q_first = qbk * kQueries + 32 * qw;
+    bf16x8_t qreg[2][KS];
+    load_q16(a, qbase, q_first, 0, l16, g, qreg[0]);
+    load_q16(a, qbase, q_first, 1, l16, g, qreg[1]);
+    // This lane's operand addresses within the wave's keys of a tile.
+    const int kidx = l16 * kRow + 8 * (g ^ l16);
+    const int vrow = 4 * g + (l16 >> 2);
+    const int vidx = vrow * kRow + (16 * (vrow & 7) + 8 * ((l16 >> 1) & 1) + 4 * (l16 & 1));
+    const int own = kKeys * kw * kRow;
+    const float c = a.c;
+    const int T = (a.Sk + kShortBN - 1) / kShortBN, full = a.Sk / kShortBN;
+    const int valid_last = a.Sk - full * kShortBN - kKeys * kw;  // <= 0: no key of the partial tile is this wave's
+
+    float m[2];
+    f32x4_t l[2], acc[2][DB];
+    // One pass over the tiles, the first one in flight or in LDS: the wave's
+    // share of it sets the reference maxima, the rest runs against them (EXACT:
+    // all with the running maximum). Ends with every wave past its last read.
+    auto pass = [&](auto exact_tag) __attribute__((always_inline)) {
+        constexpr bool EXACT = DIM != kD || decltype(exact_tag)::value;
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb) {
+            m[qb] = -INFINITY;
+            l[qb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int db = 0; db < DB; ++db) acc[qb][db] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
+        }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
+        // Tile `tile` from (kc, vc) while tile + 1 is loaded into (kn, vn).
+        auto step = [&](auto first_tag, int tile, const bf16_t *kc, const bf16_t *vc, bf16_t *kn, bf16_t *vn)
+                        __attribute__((always_inline)) {
+            load_tiles(tile + 1, kn, vn);  // past the last key: zeros (unused)
+            if constexpr (EXACT || decltype(first_tag)::value)
+                running_tile16<false, NEG, KB>(kc + own, vc + own, kKeys, qreg, kidx, vidx, g, c, m, l, acc);
+            else
+                ref_tile16<false, KB>(kc + own, vc + own, kKeys, qreg, kidx, vidx, g, c, m, l, acc);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+            __syncthreads();
+        };
+        step(std::true_type{}, 0, lds_k0, lds_v0, lds_k1, lds_v1);  // Sk >= 128 (plan_short)
+        int t = 1;
+        for (; t + 1 < full; t += 2) {
+            step(std::false_type{}, t, lds_k1, lds_v1, lds_k0, lds_v0);
+            step(std::false_type{}, t + 1, lds_k0, lds_v0, lds_k1, lds_v1);
+        }
+        if (t < full) step(std::false_type{}, t, lds_k1, lds_v1, lds_k0, lds_v0);
+        if (full < T) {  // the last, partial tile, in buffer full & 1
+            const bf16_t *kc = (full & 1 ? lds_k1 : lds_k0) + own, *vc = (full & 1 ? lds_v1 : lds_v0) + own;
+            if constexpr (EXACT)
+                running_tile16<true, NEG, KB>(kc, vc, valid_last, qreg, kidx, vidx, g, c, m, l, acc);
+            else
+                ref_tile16<true, KB>(kc, vc, valid_last, qreg, kidx, vidx, g, c, m, l, acc);
+            __syncthreads();
+        }
+    };
+    pass(std::false_type{});
+    if constexpr (DIM == kD) {
+        // Overflow against the reference maxima: redo the unit with the running
+        // maximum. The limit leaves room for the sum over the key groups, each
+        // weighted by at most 1.
+        constexpr float limit = __FLT_MAX__ / kMaxSplit;
+        bool finite = den_total(l[0], acc[0], l16) < limit && den_total(l[1], acc[1], l16) < limit;
+#pragma unroll
+        for (int qb = 0; qb < 2; ++qb)
+#pragma unroll
+            for (int db = 0; db < DB; ++db)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) finite = finite && fabsf(acc[qb][db][i]) < limit;
+        const bool wave_bad = __builtin_amdgcn_ballot_w64(!finite) != 0;
+        if (lane == 0) wave_overflow[wave] = wave_bad ? 1 : 0;
+        __syncthreads();
+        int any_bad = 0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) any_bad |= wave_overflow[w];
+        if (any_bad) {
+            load_tiles(0, lds_k0, lds_v0);
+            pass(std::true_type{});
+        }
+    }
+
+    // The key groups' partial results go over the tile buffers: 64 queries'
+    // O of a group as [64][32 chunks of 4 dims] floats in one buffer, chunk ch
+    // of query r at slot ch ^ (r & 15).
+    float *const bufs[4] = {reinterpret_cast<float *>(lds_k0), reinterpret_cast<float *>(lds_k1),
+                            reinterpret_cast<float *>(lds_v0), reinterpret_cast<float *>(lds_v1)};
+    const int at = kw * (QW / 2) + qw / 2;  // this wave's buffer
+    float *part = at == 0 ? bufs[0] : at == 1 ? bufs[1] : at == 2 ? bufs[2] : bufs[3];
+#pragma unroll
+    for (int qb = 0; qb < 2; ++qb) {
+        const int r = 32 * (qw % 2) + 16 * qb + l16;
+        const float den = den_total(l[qb], acc[qb], l16);
+        if (g == 0) state[kw][32 * qw + 16 * qb + l16] = float2{m[qb], den};
+#pragma unroll
+        for (int db = 0; db < DB; ++db)
+            *reinterpret_cast<float4 *>(part + r * kD + 4 * ((4 * db + g) ^ l16)) =
+                float4{acc[qb][db][0], acc[qb][db][1], acc[qb][db][2], acc[qb][db][3]};
+    }
+    __syncthreads();
+    // Thread t finishes chunks t % 8 + 8 j of query t / 8 of each 64 (no
+    // barrier below).
+    const int r = static_cast<int>(threadIdx.x) >> 3, j0 = static_cast<int>(threadIdx.x) & 7;
+#pragma unroll
+    for (int half = 0; half < QW / 2; ++half) {
+        const int query = qbk * kQueries + 64 * half + r;
+        if (query >= a.Sq) break;
+        float2 st[kGroups];
+        float m_all = -INFINITY;
+#pragma unroll
+        for (int p = 0; p < kGroups; ++p) {
+            st[p] = state[p][64 * half + r];
+            m_all = fmaxf(m_all, st[p].x);
+        }
+        float w[kGroups], den = 0.0f;
+#pragma unroll
+        for (int p = 0; p < kGroups; ++p) {
+            w[p] = __builtin_amdgcn_exp2f(st[p].x - m_all);
+            den += st[p].y * w[p];
+        }
+        const float inv = __fdiv_rn(1.0f, den);
+        bf16_t *orow = obase + static_cast<int64_t>(query) * a.os[2];
+#pragma unroll
+        for (int j = 0; j < (DIM / 4 + 7) / 8; ++j) {
+            const int ch = j0 + 8 * j;
+            if (DIM % 32 != 0 && ch >= DIM / 4) break;
+            float4 sum = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int p = 0; p < kGroups; ++p) {
+                const float4 x = *reinterpret_cast<const float4 *>(bufs[p * (QW / 2) + half] + r * kD + 4 * (ch ^ (r & 15)));
+                sum.x += w[p] * x.x;
+                sum.y += w[p] * x.y;
+                sum.z += w[p] * x.z;
+                sum.w += w[p] * x.w;
+            }
+            uint2 o;
+            o.x = pack2(sum.x * inv, sum.y * inv);
+            o.y = pack2(sum.z * inv, sum.w * inv);
+            *reinterpret_cast<uint2 *>(orow + 4 * ch) = o;
+        }
+    }
+}
+
 // Combines the SPLIT pieces of the tail units: a 256-thread block per (tail
 // unit, 8 queries), a thread per (query, 4 dims), all SPLIT pieces' loads
 // issued together. With M = max_p m_p and w_p = 2^(m_p - M):
 // o = bf16((sum_p w_p acc_p) / (sum_p w_p l_p)), sums in piece order.
-template <int SPLIT>
+template <int SPLIT, int DIM>
 __global__ __launch_bounds__(256) void attention_merge_kernel(AttnArgs a) {
     const int u = static_cast<int>(blockIdx.x) / (kBM / 8);
     const int r = (static_cast<int>(blockIdx.x) % (kBM / 8)) * 8 + static_cast<int>(threadIdx.x) / 32;
@@ -1225,15 +1527,15 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(AttnArgs a) {
     const int qb = unit % a.qblocks, bh = unit / a.qblocks;
     const int b = bh / a.H, h = bh % a.H;
     const int query = qb * kBM + r;
-    if (query >= a.Sq) return;  // no barrier below
+    if (query >= a.Sq || d4 >= DIM / 4) return;  // no barrier below
     const int64_t slot0 = static_cast<int64_t>(u) * SPLIT;
-    const float *ml = a.ws + static_cast<int64_t>(a.n_tail) * SPLIT * kWsSlotAcc;
+    const float *ml = a.ws + static_cast<int64_t>(a.n_tail) * SPLIT * ws_slot_acc(DIM);
     float2 st[SPLIT];
     float4 part[SPLIT];
 #pragma unroll
     for (int p = 0; p < SPLIT; ++p) {
         st[p] = *reinterpret_cast<const float2 *>(ml + (slot0 + p) * kWsSlotMl + 2 * r);
-        part[p] = *reinterpret_cast<const float4 *>(a.ws + (slot0 + p) * kWsSlotAcc + r * kD + 4 * d4);
+        part[p] = *reinterpret_cast<const float4 *>(a.ws + (slot0 + p) * ws_slot_acc(DIM) + r * DIM + 4 * d4);
     }
     float m_all = st[0].x;
 #pragma unroll
@@ -1298,6 +1600,7 @@ namespace {
 // taken when the model saves at least 3%.
 struct SplitPlan {
     int n_full = 0, n_tail = 0, split = 1;
+    double cost = 1.0;  // of the split launch, in unit-times
 };
 
 constexpr double kRoundFloor = 0.85;
@@ -1307,7 +1610,7 @@ double round_time(int64_t busy, int n_cu) {
     return f > kRoundFloor ? f : kRoundFloor;
 }
 
-SplitPlan plan_split(int64_t units, int64_t tiles, int n_cu) {
+SplitPlan plan_split(int64_t units, int64_t tiles, int n_cu, int dim) {
     SplitPlan plan;
     plan.n_full = static_cast<int>(units);
     if (n_cu <= 0 || units <= 0 || units % n_cu == 0) return plan;
@@ -1317,7 +1620,7 @@ SplitPlan plan_split(int64_t units, int64_t tiles, int n_cu) {
     for (int s = 2; s <= kMaxSplit && tiles >= 8 * s; ++s) {
         const int64_t pieces = r * s;
         const double piece = static_cast<double>((tiles + s - 1) / s) / static_cast<double>(tiles);
-        const double merge = (static_cast<double>(pieces) * kWsSlotBytes / 3.5e12 + 5e-6) / (tiles * 1.8e-6);
+        const double merge = (static_cast<double>(pieces) * ws_slot_bytes(dim) / 3.5e12 + 5e-6) / (tiles * 1.8e-6);
         const double t = static_cast<double>(rounds) +
                          piece * (static_cast<double>(pieces / n_cu) + (pieces % n_cu ? round_time(pieces % n_cu, n_cu) : 0.0)) +
                          merge;
@@ -1329,6 +1632,7 @@ SplitPlan plan_split(int64_t units, int64_t tiles, int n_cu) {
     if (plan.split == 1 || best > 0.97 * unsplit) return SplitPlan{static_cast<int>(units), 0, 1};
     plan.n_full = static_cast<int>(rounds * n_cu);
     plan.n_tail = static_cast<int>(r);
+    plan.cost = best;
     return plan;
 }
 
@@ -1369,14 +1673,57 @@ SmallPlan plan_small(int64_t heads, int64_t Sq, int n_cu) {
 }
 
 
+// Launches of at most one round of 256-query units: 64- or 128-query units with
+// the keys split over a workgroup's waves (attention16_short_kernel) where the
+// times below say so. Fitted to launches of 7 to 56 heads over 64 to 4096
+// tokens, D = 128 and 72, in us: a round of 256-query units takes 9 + 1.3 per
+// 64-key tile (1.45 on a full chip), of 128-query units 7 + 1.58 and of 64-query
+// units 7 + 1.1 per 128-key tile. At 14 heads (units of 256 / 128 / 64 queries,
+// the best key split over workgroups): S = 256: 14.4 / 10.6 / 9.2, 15.4; 1024:
+// 29.7 / 19.0 / 15.1, 24.3; 2048: 50.6 / 32.8 / 43.9, 41.1; 3000: 70.8 / 85.9 /
+// 90.5, 82.2. Returns the query waves per workgroup (2 or 4), 0 for none.
+int plan_short(int64_t heads, int64_t Sq, int64_t Sk, int n_cu, int dim) {
+    if (n_cu <= 0) return 0;
+    auto rounds = [&](int64_t bm) { return static_cast<double>((heads * ((Sq + bm - 1) / bm) + n_cu - 1) / n_cu); };
+    const int64_t units = heads * ((Sq + kBM - 1) / kBM), tiles = (Sk + kBN - 1) / kBN;
+    // The kernel needs one whole 128-key tile (shorter sequences gain nothing:
+    // 65 keys 8.0 against 8.2 us, 128 keys 9.0 against 8.2 us).
+    if (units > n_cu || Sk < kShortBN) return 0;
+    const SplitPlan split = plan_split(units, tiles, n_cu, dim);
+    const double big = 9.0 + tiles * (split.split > 1 ? 1.45 * split.cost : 1.3);
+    const double steps = static_cast<double>((Sk + kShortBN - 1) / kShortBN);
+    const double t2 = 7.0 + 1.1 * steps * rounds(64), t4 = 7.0 + 1.58 * steps * rounds(128);
+    if ((t2 < t4 ? t2 : t4) > 0.97 * big) return 0;
+    return t2 < t4 ? 2 : 4;
+}
+
+// The key-split launch and its merge.
+template <int DIM>
+int launch_split(const AttnArgs &a, bool neg, unsigned grid, hipStream_t st) {
+    if (neg)
+        attention16_kernel<true, true, DIM><<<grid, kThreadsWG, 0, st>>>(a);
+    else
+        attention16_kernel<false, true, DIM><<<grid, kThreadsWG, 0, st>>>(a);
+    const unsigned gm = static_cast<unsigned>(a.n_tail * (kBM / 8));
+    switch (a.split) {
+#define H3_MERGE(S) \
+    case S: attention_merge_kernel<S, DIM><<<gm, 256, 0, st>>>(a); break;
+        H3_MERGE(2) H3_MERGE(3) H3_MERGE(4) H3_MERGE(5) H3_MERGE(6) H3_MERGE(7) H3_MERGE(8)
+#undef H3_MERGE
+        default: return kInvalid;
+    }
+    return launch_status();
+}
+
 // The launcher of both numerics: fp32_qk (logits scaled by c = scale log2 e in
 // fp32) and bf16_prescale (q rounded to bf16(c q) before the product).
-// workspace (fp32_qk, D = 128, may be null): bytes for the key split of the
-// last round; too small for the planned split (empty included), the launch
-// runs unsplit.
+// workspace (fp32_qk, may be null): bytes for the key split of the last round;
+// too small for the planned split (empty included), the launch runs unsplit.
+// planned: a launch of few units may also run as 64-query units
+// (attention16_short_kernel).
 int launch_attention(NineToothedStream stream, NineToothedTensor q, NineToothedTensor k, NineToothedTensor v,
                      NineToothedTensor scale, NineToothedTensor o, bool prescale, int64_t dim,
-                     const NineToothedTensor *workspace = nullptr) {
+                     const NineToothedTensor *workspace = nullptr, bool planned = false) {
     View<4> qv, kv, vv, ov;
     View<1> wv;
     double sc;
@@ -1443,12 +1790,23 @@ int launch_attention(NineToothedStream stream, NineToothedTensor q, NineToothedT
     hipStream_t st = as_stream(stream);
     const bool neg = a.c < 0.0f && !prescale;  // the loop's max runs over c * s
     int n_cu = 0;
-    if (buf && dim == kD) {
+    if (buf) {
         int dev = 0;
         const hipError_t e = hipStreamGetDevice(st, &dev);
         if (e != hipSuccess) return static_cast<int>(e);
         n_cu = device_cus(dev);
-        const SmallPlan sp = plan_small(static_cast<int64_t>(a.B) * a.H, a.Sq, n_cu);
+        const int qw = planned ? plan_short(static_cast<int64_t>(a.B) * a.H, a.Sq, a.Sk, n_cu, static_cast<int>(dim)) : 0;
+        if (qw != 0) {
+            a.qblocks = (a.Sq + 32 * qw - 1) / (32 * qw);
+            const unsigned gs = static_cast<unsigned>(a.B * a.H * a.qblocks);
+#define H3_SHORT(N, D, Q) \
+    if (neg == N && dim == D && qw == Q) attention16_short_kernel<N, D, Q><<<gs, kThreadsWG, 0, st>>>(a);
+            H3_SHORT(false, 128, 2) H3_SHORT(true, 128, 2) H3_SHORT(false, 72, 2) H3_SHORT(true, 72, 2)
+            H3_SHORT(false, 128, 4) H3_SHORT(true, 128, 4) H3_SHORT(false, 72, 4) H3_SHORT(true, 72, 4)
+#undef H3_SHORT
+            return launch_status();
+        }
+        const SmallPlan sp = dim == kD ? plan_small(static_cast<int64_t>(a.B) * a.H, a.Sq, n_cu) : SmallPlan{};
         if (sp.use) {
             a.n_big = sp.n_big;
             a.n_small = sp.n_small;
@@ -1465,35 +1823,29 @@ int launch_attention(NineToothedStream stream, NineToothedTensor q, NineToothedT
             return launch_status();
         }
     }
-    if (workspace != nullptr && buf && dim == kD && !prescale && wv.shape[0] > 0) {
-        const SplitPlan plan = plan_split(grid, (a.Sk + kBN - 1) / kBN, n_cu);
+    if (workspace != nullptr && buf && !prescale && wv.shape[0] > 0) {
+        const SplitPlan plan = plan_split(grid, (a.Sk + kBN - 1) / kBN, n_cu, static_cast<int>(dim));
         const int64_t pieces = static_cast<int64_t>(plan.n_tail) * plan.split;
-        if (plan.split > 1 && wv.shape[0] >= pieces * kWsSlotBytes) {
+        if (plan.split > 1 && wv.shape[0] >= pieces * ws_slot_bytes(static_cast<int>(dim))) {
             a.n_full = plan.n_full;
             a.n_tail = plan.n_tail;
             a.split = plan.split;
             a.ws = reinterpret_cast<float *>(wv.data);
-            const unsigned gs = static_cast<unsigned>(plan.n_full + pieces);
-            if (neg)
-                attention16_kernel<true, true><<<gs, kThreadsWG, 0, st>>>(a);
-            else
-                attention16_kernel<false, true><<<gs, kThreadsWG, 0, st>>>(a);
-            const unsigned gm = static_cast<unsigned>(plan.n_tail * (kBM / 8));
-            switch (plan.split) {
-#define H3_MERGE(S) \
-    case S: attention_merge_kernel<S><<<gm, 256, 0, st>>>(a); break;
-                H3_MERGE(2) H3_MERGE(3) H3_MERGE(4) H3_MERGE(5) H3_MERGE(6) H3_MERGE(7) H3_MERGE(8)
-#undef H3_MERGE
-                default: return kInvalid;
-            }
-            return launch_status();
+            return dim == kD ? launch_split<kD>(a, neg, static_cast<unsigned>(plan.n_full + pieces), st)
+                             : launch_split<72>(a, neg, static_cast<unsigned>(plan.n_full + pieces), st);
         }
     }
-    if (buf && dim == kD) {
-        if (neg)
-            attention16_kernel<true, false><<<g, kThreadsWG, 0, st>>>(a);
-        else
-            attention16_kernel<false, false><<<g, kThreadsWG, 0, st>>>(a);
+    // D = 72 with a fifth or more of the CUs idle: the chip then runs at its top
+    // clock, where the 32x32x16 kernel's tiles take 1.27 us against 1.42 us
+    // (144 to 192 units; 63.3 against 68.9 us at 16 heads, S = 3000), while on a
+    // full chip, under its power limit, the 16x16x32 products win (S = 4096:
+    // 93.3 against 97.3 us; 240 units: 81.9 against 83.4 us).
+    const bool idle72 = dim != kD && 5 * grid <= 4 * static_cast<int64_t>(n_cu);
+    if (buf && !idle72) {
+#define H3_ATTN16(N, D) \
+    if (neg == N && dim == D) attention16_kernel<N, false, D><<<g, kThreadsWG, 0, st>>>(a);
+        H3_ATTN16(false, 128) H3_ATTN16(true, 128) H3_ATTN16(false, 72) H3_ATTN16(true, 72)
+#undef H3_ATTN16
         return launch_status();
     }
 #define H3_ATTN(N, B, D, G) \
@@ -1522,15 +1874,37 @@ extern "C" NineToothedResult launch_h3_full_attention_ws(NineToothedStream strea
     return launch_attention(stream, q, k, v, scale, o, false, kD, &workspace);
 }
 
-extern "C" int64_t h3_full_attention_workspace_bytes(int64_t B, int64_t H, int64_t Sq, int64_t Sk) {
+namespace {
+
+int64_t workspace_bytes(int64_t B, int64_t H, int64_t Sq, int64_t Sk, int dim, bool planned) {
     if (B <= 0 || H <= 0 || Sq <= 0 || Sk <= 0 || Sq > kMaxSeqLen || Sk > kMaxSeqLen) return 0;
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess) return -1;
+    const int n_cu = device_cus(dev);
     const int64_t units = B * H * ((Sq + kBM - 1) / kBM);
     if (units > std::numeric_limits<int32_t>::max()) return 0;
-    if (plan_small(B * H, Sq, device_cus(dev)).use) return 0;  // the 192-query last round needs none
-    const SplitPlan plan = plan_split(units, (Sk + kBN - 1) / kBN, device_cus(dev));
-    return plan.split > 1 ? static_cast<int64_t>(plan.n_tail) * plan.split * kWsSlotBytes : 0;
+    if (planned && plan_short(B * H, Sq, Sk, n_cu, dim) != 0) return 0;
+    if (dim == kD && plan_small(B * H, Sq, n_cu).use) return 0;  // the 192-query last round needs none
+    const SplitPlan plan = plan_split(units, (Sk + kBN - 1) / kBN, n_cu, dim);
+    return plan.split > 1 ? static_cast<int64_t>(plan.n_tail) * plan.split * ws_slot_bytes(dim) : 0;
+}
+
+}  // namespace
+
+extern "C" int64_t h3_full_attention_workspace_bytes(int64_t B, int64_t H, int64_t Sq, int64_t Sk) {
+    return workspace_bytes(B, H, Sq, Sk, kD, false);
+}
+
+extern "C" int64_t h3_attention_planned_workspace_bytes(int64_t B, int64_t H, int64_t Sq, int64_t Sk, int64_t D) {
+    return D == kD || D == 72 ? workspace_bytes(B, H, Sq, Sk, static_cast<int>(D), true) : 0;
+}
+
+extern "C" NineToothedResult launch_h3_attention_planned(NineToothedStream stream, NineToothedTensor q,
+                                                         NineToothedTensor k, NineToothedTensor v,
+                                                         NineToothedTensor scale, NineToothedTensor o,
+                                                         NineToothedTensor workspace) {
+    const bool vision = q.shape != nullptr && q.shape[3] == 72;
+    return launch_attention(stream, q, k, v, scale, o, false, vision ? 72 : kD, &workspace, true);
 }
 
 extern "C" NineToothedResult launch_h3_vision_attention_72(NineToothedStream stream, NineToothedTensor q,

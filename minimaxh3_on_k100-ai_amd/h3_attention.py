@@ -16,12 +16,13 @@ Numerics (tools/h3_attention.py:25-101):
     masked, so the three coincide.
   - "bf16_prescale" (:87-101): q enters the product as bf16(fp32(scale log2 e) q)
     and the logits are used unscaled (launch_h3_full_attention_bf16_prescale).
-  At head_dim 128 the softmax's stabilising maximum is the first key tile's,
+  The softmax's stabilising maximum is the first key tile's,
   kept for the rest of a 256-query unit (the unit is recomputed with the
   running maximum if anything overflows against it), and the denominator
   sums the same bf16-rounded P that multiplies V. The reference rescales at
   every new running maximum and sums P in fp32; the results agree within the
-  operator's tolerance. head_dim 72 keeps the reference's order.
+  operator's tolerance. head_dim 72 takes the same order; K/V views outside
+  the 16-byte tile path keep the reference's.
 head_dim 128 (the DiT's) and 72 (the Qwen vision tower's, launcher
 launch_h3_vision_attention_72 as in scripts/build_h3_attention.py:23-24) are
 built; as in the reference, a factory runs only tensors of its own head_dim.
@@ -56,11 +57,11 @@ def make_attention(block_m=128, block_n=32, num_warps=4, num_stages=1, caller="t
                    archs=None, backend_options=None, kernel_name="h3_full_attention", numerics="fp32_qk",
                    head_dim=128, dtype=None, *, split_last_round=True):
     """The reference's factory (tools/h3_attention.py:104-121). split_last_round
-    (fp32_qk numerics, head_dim 128; no counterpart in the reference): when the
-    launch's last round of 256-query workgroups is only partly filled, its
-    units are split along the keys (launch_h3_full_attention_ws) with a
-    workspace from torch's caching allocator; False always runs the unsplit
-    launch_h3_full_attention."""
+    (fp32_qk numerics; no counterpart in the reference): when the launch's last
+    round of 256-query workgroups is only partly filled, its units are split
+    along the keys (launch_h3_attention_planned), over workgroups with a
+    workspace from torch's caching allocator or over the waves of smaller
+    units; False always runs the unsplit launch."""
     if head_dim <= 0:
         raise ValueError("head_dim must be positive")
     if head_dim not in (128, 72):
@@ -77,7 +78,7 @@ def make_attention(block_m=128, block_n=32, num_warps=4, num_stages=1, caller="t
     else:
         entry = "launch_h3_full_attention_bf16_prescale" if numerics == "bf16_prescale" else "launch_h3_full_attention"
 
-    split = split_last_round and entry == "launch_h3_full_attention"
+    split = split_last_round and numerics != "bf16_prescale"
     plans: dict = {}  # (device, B, H, Sq, Sk) -> workspace bytes
 
     def kernel(q, k, v, scale, out):
@@ -91,12 +92,11 @@ def make_attention(block_m=128, block_n=32, num_warps=4, num_stages=1, caller="t
             nbytes = plans.get(key)
             if nbytes is None:
                 with torch.cuda.device(device):
-                    nbytes = plans[key] = _lib.attention_workspace_bytes(*key[1:])
-            if nbytes > 0:
-                ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
-                _lib.launch("launch_h3_full_attention_ws", device, _lib.tensor(q), _lib.tensor(k), _lib.tensor(v),
-                            _lib.scalar(scale), _lib.tensor(out), _lib.tensor(ws))
-                return
+                    nbytes = plans[key] = _lib.attention_planned_workspace_bytes(*key[1:], head_dim)
+            ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
+            _lib.launch("launch_h3_attention_planned", device, _lib.tensor(q), _lib.tensor(k), _lib.tensor(v),
+                        _lib.scalar(scale), _lib.tensor(out), _lib.tensor(ws))
+            return
         _lib.launch(entry, device, _lib.tensor(q), _lib.tensor(k), _lib.tensor(v), _lib.scalar(scale),
                     _lib.tensor(out))
 

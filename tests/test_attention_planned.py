@@ -1,0 +1,111 @@
+"""launch_h3_attention_planned: the plan's 64- and 128-query units with the keys
+split over a workgroup's waves (attention16_short_kernel), against the float64
+oracle, and the entry point's argument checks."""
+from __future__ import annotations
+
+import ctypes
+
+import pytest
+import torch
+
+from conftest import attention_error
+from test_attention_gpu import MAX_ABS, REL_RMS, _bhsd, _dominant_keys
+
+BF = torch.bfloat16
+_BUF = ctypes.create_string_buffer(1 << 16)
+
+
+@pytest.mark.parametrize("shapes", [
+    ([1, 2, 8, 64], [1, 2, 8, 64], [1, 2, 8, 64], [0]),    # head dim
+    ([1, 2, 8, 72], [1, 2, 8, 128], [1, 2, 8, 72], [0]),   # k and q differ
+    ([1, 2, 8, 128], [1, 2, 0, 128], [1, 2, 8, 128], [0]),  # no keys
+    ([1, 2, 8, 128], [1, 2, 8, 128], [1, 2, 9, 128], [0]),  # out length
+])
+def test_planned_entry_rejects_bad_shapes(shapes):
+    import importlib
+    L = importlib.import_module("minimaxh3_on_k100-ai_amd")._lib
+
+    def t(shape):
+        strides = [1] * len(shape)
+        for i in range(len(shape) - 2, -1, -1):
+            strides[i] = strides[i + 1] * max(shape[i + 1], 1)
+        return L.raw_tensor((ctypes.addressof(_BUF) + 255) & ~255, shape, strides)
+
+    q, k, o, ws = (t(s) for s in shapes)
+    assert L.call("launch_h3_attention_planned", 0, q, k, k, L.scalar(0.1), o, ws) == L.HIP_ERROR_INVALID_VALUE
+    assert L.attention_planned_workspace_bytes(0, 1, 5, 5, 128) == 0
+    assert L.attention_planned_workspace_bytes(1, 1, 5, 5, 64) == 0
+
+
+def _kernels(fn):
+    from torch.profiler import ProfilerActivity, profile
+    with profile(activities=[ProfilerActivity.CUDA]) as prof:
+        fn()
+        torch.cuda.synchronize()
+    return [e.name for e in prof.events() if "attention" in e.name]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [128, 72])
+@pytest.mark.parametrize("B,H,Sq,Sk,scale,QW", [
+    (1, 3, 1, 129, 0.1, 2),        # one query; one key past a tile: waves without keys in the second
+    (2, 3, 63, 255, 0.1, 2),       # the last query of a unit and the last key of a tile missing
+    (1, 2, 64, 128, -0.1, 2),      # one whole tile, one whole unit, negative scale
+    (1, 2, 65, 193, 0.1, 2),       # one query past a unit
+    (1, 2, 130, 1000, 0.0, 2),     # zero scale; the last wave of the partial tile without keys
+    (2, 7, 1200, 1100, 0.1, 4),    # 266 units of 64 queries on 256 CUs: 128-query units
+    (1, 16, 1537, 257, -0.1, 4),   # 13 units a head, the last of one query
+])
+def test_short_units_match_fp64(pkg, oracle, device, D, B, H, Sq, Sk, scale, QW):
+    """Both unit sizes at the edges of their tiles, in buffers whose
+    neighbouring head is NaN: within the operator's bar of float64, two
+    launches bitwise equal, doubling V doubles the output bitwise."""
+    gen = torch.Generator("cpu").manual_seed(Sq * 5 + Sk + D)
+    bufs = [torch.full((B, s, H + 1, D), float("nan")) for s in (Sq, Sk, Sk)]
+    for b in bufs:
+        b[:, :, :H] = torch.randn(b[:, :, :H].shape, generator=gen)
+    q, k, v = (_bhsd(b.to(BF)[:, :, :H]) for b in bufs)
+    qd, kd, vd = (_bhsd(b.to(BF).to(device)[:, :, :H]) for b in bufs)
+    out = torch.full((B, Sq, H, D), float("nan"), dtype=BF, device=device)
+    out1, out2 = torch.full_like(out, float("nan")), torch.full_like(out, float("nan"))
+    attn = pkg.make_attention(head_dim=D)
+    names = _kernels(lambda: attn(qd, kd, vd, scale, _bhsd(out)))
+    if torch.cuda.get_device_properties(device).multi_processor_count == 256:
+        neg = "true" if scale < 0 else "false"
+        assert len(names) == 1 and f"attention16_short_kernel<{neg}, {D}, {QW}>" in names[0], names
+    attn(qd, kd, vd, scale, _bhsd(out1))
+    attn(qd, kd, vd * 2, scale, _bhsd(out2))
+    torch.cuda.synchronize()
+    mx, rel = attention_error(_bhsd(out).cpu(), oracle.attention(q, k, v, scale))
+    assert mx <= MAX_ABS and rel <= REL_RMS, (mx, rel)
+    assert torch.equal(out, out1) and torch.equal(out2, out * 2)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [128, 72])
+@pytest.mark.parametrize("case", ["overflow", "dominated", "denominator", "huge_values"])
+def test_short_units_reference_maximum(pkg, oracle, device, D, case):
+    """A key far above the first tile's maxima, in a later tile and one key
+    group: exact where its weight dominates, recomputed with the running
+    maximum where p, a denominator or O leaves its range."""
+    keys = [320, 324, 328, 332] if case == "denominator" else [333]
+    q, k, v = _dominant_keys(700, keys, 127.0, 0.25 if case == "denominator" else 1.96875)
+    if case == "overflow":
+        k[0, 0, 333, 0] = 100.0
+    elif case == "dominated":
+        k[0, 0, 333, 0] = 24.0
+    elif case == "huge_values":
+        k[0, 0, 300:, 0] = 10.0
+        v = (v.float().sign() * 1e33 + v.float() * 1e31).to(BF)
+    q, k, v = (t[..., :D].contiguous() for t in (q, k, v))
+    scale = 128 ** -0.5
+    want = oracle.attention(q.double(), k.double(), v.double(), scale)
+    out = torch.full(q.shape, float("nan"), dtype=BF, device=device)
+    pkg.make_attention(head_dim=D)(q.to(device), k.to(device), v.to(device), scale, out)
+    torch.cuda.synchronize()
+    got = out.cpu()
+    assert torch.isfinite(got.float()).all()
+    if case in ("overflow", "dominated"):
+        assert torch.equal(got, torch.full_like(got, 1.96875))
+    rel = float((got.double() - want).norm() / want.norm())
+    assert rel <= REL_RMS, rel
