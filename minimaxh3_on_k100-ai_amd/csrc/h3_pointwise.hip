@@ -331,13 +331,12 @@ __global__ __launch_bounds__(kThreads) void rms_lanes_kernel(RmsArgs a) {
     }
 }
 
-// Rows of 64 < W8 <= 64 * G groups with per-row modulation (or a generic
-// layout): one row per wave. Lane l takes groups l + 64k (k < G) and keeps four
-// partial sums, one for each of the threads l + 64w (w = k mod 4) of the
-// 256-thread order, which it reproduces exactly. Weight, scale and shift come
-// in batches of four groups, each batch's loads issued before the previous
-// batch's stores.
-template <int G, bool VEC, int MODE>
+// Rows of 64 < W8 <= 64 * G groups in a generic layout: one row per wave. Lane l
+// takes groups l + 64k (k < G) and keeps four partial sums, one for each of the
+// threads l + 64w (w = k mod 4) of the 256-thread order, which it reproduces
+// exactly. Weight, scale and shift come in batches of four groups, each batch's
+// loads issued before the previous batch's stores.
+template <int G, int MODE>
 __global__ __launch_bounds__(kThreads) void rms_wave_kernel(RmsArgs a) {
     constexpr int kChunk = 4;
     constexpr int kChunks = (G + kChunk - 1) / kChunk;
@@ -352,10 +351,10 @@ __global__ __launch_bounds__(kThreads) void rms_wave_kernel(RmsArgs a) {
 #pragma unroll
     for (int k = 0; k < G; ++k) {
         const int c0 = clamp_group(lane + 64 * k, W8) * 8;
-        v[k] = load_group<VEC, true>(row_ptr(a.x, b, s), a.x.sw, c0, a.W);
+        v[k] = load_group<false, true>(row_ptr(a.x, b, s), a.x.sw, c0, a.W);
         if constexpr (MODE == kGatedRmsModulate) {
-            gv[k] = load_group<VEC>(row_ptr(a.gate, mb, ms), a.gate.sw, c0, a.W);
-            yv[k] = load_group<VEC, true>(row_ptr(a.y, b, s), a.y.sw, c0, a.W);
+            gv[k] = load_group<false>(row_ptr(a.gate, mb, ms), a.gate.sw, c0, a.W);
+            yv[k] = load_group<false, true>(row_ptr(a.y, b, s), a.y.sw, c0, a.W);
         }
     }
     __builtin_amdgcn_sched_barrier(0);  // the row's loads stay together, ahead of its arithmetic
@@ -364,10 +363,10 @@ __global__ __launch_bounds__(kThreads) void rms_wave_kernel(RmsArgs a) {
 #pragma unroll
         for (int j = 0; j < kChunk; ++j) {
             const int c0 = clamp_group(lane + 64 * (c * kChunk + j), W8) * 8;
-            wv[c & 1][j] = load_group<VEC>(a.w, a.w_stride, c0, a.W);
+            wv[c & 1][j] = load_group<false>(a.w, a.w_stride, c0, a.W);
             if constexpr (MODE != kRms) {
-                scv[c & 1][j] = load_group<VEC>(row_ptr(a.scale, mb, ms), a.scale.sw, c0, a.W);
-                shv[c & 1][j] = load_group<VEC>(row_ptr(a.shift, mb, ms), a.shift.sw, c0, a.W);
+                scv[c & 1][j] = load_group<false>(row_ptr(a.scale, mb, ms), a.scale.sw, c0, a.W);
+                shv[c & 1][j] = load_group<false>(row_ptr(a.shift, mb, ms), a.shift.sw, c0, a.W);
             }
         }
     };
@@ -378,7 +377,7 @@ __global__ __launch_bounds__(kThreads) void rms_wave_kernel(RmsArgs a) {
         const int g = lane + 64 * k;
         v[k] = rms_phase1<MODE>(v[k], gv[k], yv[k], g < W8, part[k & 3]);
         if constexpr (MODE == kGatedRmsModulate)
-            if (g < W8) store_group<VEC, true>(row_ptr_w(a.residual, b, s), a.residual.sw, g * 8, a.W, v[k]);
+            if (g < W8) store_group<false, true>(row_ptr_w(a.residual, b, s), a.residual.sw, g * 8, a.W, v[k]);
         keep_packed(v[k]);
     }
     const float total = (fold_lanes<64>(part[0]) + fold_lanes<64>(part[2])) +
@@ -392,7 +391,7 @@ __global__ __launch_bounds__(kThreads) void rms_wave_kernel(RmsArgs a) {
             const int k = c * kChunk + j, g = lane + 64 * k;
             if (k < G) {
                 const U4 o = rms_phase2<MODE>(v[k], r, wv[c & 1][j], factor_of(scv[c & 1][j]), shv[c & 1][j]);
-                if (g < W8) store_group<VEC, true>(row_ptr_w(a.out, b, s), a.out.sw, g * 8, a.W, o);
+                if (g < W8) store_group<false, true>(row_ptr_w(a.out, b, s), a.out.sw, g * 8, a.W, o);
             }
         }
     }
@@ -420,16 +419,19 @@ __device__ __forceinline__ void stage_vectors(const RmsArgs &a, int64_t b, int W
 // the rows in flight are close together in memory. After a row's own loads the
 // only global accesses are its stores.
 //
-// EXACT: W8 = 64 G, so no group is clamped or masked; the row's addresses are
+// EXACT: W8 = 64 G, so no group is clamped or masked; otherwise
+// 64 (G - 1) < W8 < 64 G and only the last group is. The row's addresses are
 // then one base and constant offsets, the kernel is held to 80 VGPRs (at
-// G = 14 it fits them without spilling), and three
+// G = 14 it fits them without spilling; 15 and 16 take 96, a partial last group
+// 74 to 96), and up to three
 // 512-thread blocks share a CU (24 waves, 6144 rows in flight over the chip):
-// measured 46.5 against 49.5 us for the clamped form at two blocks per CU
-// (RMSNorm + AdaLN at [8192, 7168]). The EXACT kernel over 2 or 4 blocks per CU
-// measured 51 us; 16-byte aligned LDS reads of the staged rows (ds_read_b128
+// RMSNorm + AdaLN at [8192, 7168] 46.1 us. Against every group clamped, G
+// rounded up to an even number and two blocks per CU: 49.5 us there, and 77.4
+// against 74.4 us at [18000, 5376]. G = 16 held to 80 VGPRs spilled 74 of them:
+// 36.0 against 28.1 us at [4000, 8192]. 16-byte aligned LDS reads of the staged rows (ds_read_b128
 // instead of ds_read2_b32 pairs) made it spill 284 bytes and cost 2.4x.
 template <int G, int MODE, int THREADS, bool EXACT>
-__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(EXACT ? 6 : 1)))
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(EXACT ? (G <= 14 ? 6 : 5) : (G <= 12 ? 5 : 4))))
 void rms_staged_kernel(RmsArgs a) {
     static_assert(MODE != kGatedRmsModulate, "the gated mode runs as rms_stream_kernel");
     extern __shared__ U4 staged[];
@@ -437,18 +439,15 @@ void rms_staged_kernel(RmsArgs a) {
     const int64_t b = blockIdx.y;
     const int lane = threadIdx.x & 63;
     const int64_t step = static_cast<int64_t>(gridDim.x) * (THREADS / 64);
-    auto group = [&](int g) { return EXACT ? g : clamp_group(g, W8); };
+    auto group = [&](int k) { return EXACT || k < G - 1 ? lane + 64 * k : clamp_group(lane + 64 * k, W8); };
     U4 v[G], yv[G];
     auto load_row = [&](int64_t s) {
 #pragma unroll
         for (int k = 0; k < G; ++k) {
-            const int c0 = group(lane + 64 * k) * 8;
+            const int c0 = group(k) * 8;
             v[k] = ld16_stream(row_ptr(a.x, b, s) + c0);
             if constexpr (MODE == kGatedRmsModulate) yv[k] = ld16_stream(row_ptr(a.y, b, s) + c0);
         }
-        // The row's loads stay together, ahead of its arithmetic (EXACT's
-        // constant offsets keep them together without the barrier, in fewer
-        // registers).
         if constexpr (!EXACT) __builtin_amdgcn_sched_barrier(0);
     };
     int64_t s = static_cast<int64_t>(blockIdx.x) * (THREADS / 64) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -462,12 +461,12 @@ void rms_staged_kernel(RmsArgs a) {
         float part[4] = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
         for (int k = 0; k < G; ++k) {
-            const int g = lane + 64 * k, gc = group(g);
+            const int g = lane + 64 * k, gc = group(k);
             U4 gv{};
             if constexpr (MODE == kGatedRmsModulate) gv = lg[gc];
-            v[k] = rms_phase1<MODE>(v[k], gv, yv[k], EXACT || g < W8, part[k & 3]);
+            v[k] = rms_phase1<MODE>(v[k], gv, yv[k], EXACT || k < G - 1 || g < W8, part[k & 3]);
             if constexpr (MODE == kGatedRmsModulate)
-                if (EXACT || g < W8) st16_stream(row_ptr_w(a.residual, b, s) + g * 8, v[k]);
+                if (EXACT || k < G - 1 || g < W8) st16_stream(row_ptr_w(a.residual, b, s) + g * 8, v[k]);
             keep_packed(v[k]);
         }
         const float total = (fold_lanes<64>(part[0]) + fold_lanes<64>(part[2])) +
@@ -475,14 +474,14 @@ void rms_staged_kernel(RmsArgs a) {
         const float r = rms_reciprocal(total, a.W, a.eps_bf);
 #pragma unroll
         for (int k = 0; k < G; ++k) {
-            const int g = lane + 64 * k, gc = group(g);
+            const int g = lane + 64 * k, gc = group(k);
             U4 kv{}, shv{};
             if constexpr (MODE != kRms) {
                 kv = lk[gc];
                 shv = lsh[gc];
             }
             const U4 o = rms_phase2<MODE>(v[k], r, lw[gc], kv, shv);
-            if (EXACT || g < W8) st16_stream(row_ptr_w(a.out, b, s) + g * 8, o);
+            if (EXACT || k < G - 1 || g < W8) st16_stream(row_ptr_w(a.out, b, s) + g * 8, o);
         }
     }
 }
@@ -502,7 +501,8 @@ void rms_staged_kernel(RmsArgs a) {
 // shift from the tables (L2) instead. The launch bound keeps two blocks
 // resident per CU up to G = 14 (W = 7168).
 //
-// EXACT: W8 = 64 G, so no group is clamped or masked.
+// EXACT: W8 = 64 G, so no group is clamped or masked; otherwise
+// 64 (G - 1) < W8 < 64 G and only the last group is.
 template <int G, int THREADS, bool EXACT>
 __global__ __launch_bounds__(THREADS, G <= 14 ? 4 : 3) void rms_modulate_indexed_kernel(RmsArgs a) {
     constexpr int kWaves = THREADS / 64;
@@ -515,14 +515,12 @@ __global__ __launch_bounds__(THREADS, G <= 14 ? 4 : 3) void rms_modulate_indexed
     const int64_t step = static_cast<int64_t>(gridDim.x) * kWaves;
     const int64_t last = a.rows - 1;
     const uint32_t S32 = static_cast<uint32_t>(a.S);
+    auto group = [&](int k) { return EXACT || k < G - 1 ? lane + 64 * k : clamp_group(lane + 64 * k, W8); };
     U4 v[G];
     auto load_row = [&](int64_t b, int64_t s) {
 #pragma unroll
         for (int k = 0; k < G; ++k)
-            v[k] = ld16_stream(row_ptr(a.x, b, s) + (EXACT ? lane + 64 * k : clamp_group(lane + 64 * k, W8)) * 8);
-        // The row's loads stay together, ahead of its arithmetic (EXACT's
-        // constant offsets keep them together without the barrier).
-        if constexpr (!EXACT) __builtin_amdgcn_sched_barrier(0);
+            v[k] = ld16_stream(row_ptr(a.x, b, s) + group(k) * 8);
     };
     int64_t in_lds = -1;
     for (int64_t base = static_cast<int64_t>(blockIdx.x) * kWaves; base < a.rows; base += step) {
@@ -563,7 +561,7 @@ __global__ __launch_bounds__(THREADS, G <= 14 ? 4 : 3) void rms_modulate_indexed
 #pragma unroll
         for (int k = 0; k < G; ++k) {
             const U4 unused{};
-            v[k] = rms_phase1<kRmsModulate>(v[k], unused, unused, EXACT || lane + 64 * k < W8, part[k & 3]);
+            v[k] = rms_phase1<kRmsModulate>(v[k], unused, unused, EXACT || k < G - 1 || lane + 64 * k < W8, part[k & 3]);
             keep_packed(v[k]);
         }
         const float total = (fold_lanes<64>(part[0]) + fold_lanes<64>(part[2])) +
@@ -572,18 +570,18 @@ __global__ __launch_bounds__(THREADS, G <= 14 ? 4 : 3) void rms_modulate_indexed
         if (same) {
 #pragma unroll
             for (int k = 0; k < G; ++k) {
-                const int g = lane + 64 * k, gc = EXACT ? g : clamp_group(g, W8);
+                const int g = lane + 64 * k, gc = group(k);
                 const U4 o = rms_phase2<kRmsModulate>(v[k], r, lw[gc], lk[gc], lsh[gc]);
-                if (ok && (EXACT || g < W8)) st16_stream(row_ptr_w(a.out, b, s) + g * 8, o);
+                if (ok && (EXACT || k < G - 1 || g < W8)) st16_stream(row_ptr_w(a.out, b, s) + g * 8, o);
             }
         } else {
 #pragma unroll
             for (int k = 0; k < G; ++k) {
-                const int g = lane + 64 * k, gc = EXACT ? g : clamp_group(g, W8);
+                const int g = lane + 64 * k, gc = group(k);
                 const U4 kv = factor_of(ld16(row_ptr(a.scale, mine, 0) + gc * 8));
                 const U4 shv = ld16(row_ptr(a.shift, mine, 0) + gc * 8);
                 const U4 o = rms_phase2<kRmsModulate>(v[k], r, lw[gc], kv, shv);
-                if (ok && (EXACT || g < W8)) st16_stream(row_ptr_w(a.out, b, s) + g * 8, o);
+                if (ok && (EXACT || k < G - 1 || g < W8)) st16_stream(row_ptr_w(a.out, b, s) + g * 8, o);
                 __builtin_amdgcn_sched_barrier(0);  // one group's table loads at a time (registers)
             }
         }
@@ -598,51 +596,30 @@ __global__ __launch_bounds__(THREADS, G <= 14 ? 4 : 3) void rms_modulate_indexed
 // flight while a row is reduced and written), so the blocks stream a sliding
 // window of rows. The four wave partials meet in LDS (double-buffered by row
 // parity, one barrier per row).
-//
-// INDEXED: every token names its modulation row (ModIndex). The blocks walk
-// all B * S rows grid-strided; a row's index is loaded with its data (one
-// value for the whole block), and the block stages that row of the tables
-// whenever it differs from the one in LDS -- once per run of equal indices a
-// block meets, since a block's rows are in token order.
-template <int VPT, int MODE, int DEPTH, bool INDEXED>
+template <int VPT, int MODE, int DEPTH>
 __global__ __launch_bounds__(kThreads) void rms_stream_kernel(RmsArgs a) {
     extern __shared__ U4 staged[];
     __shared__ float red[2][kThreads / 64];
     const int W8 = (a.W + 7) / 8;
-    const int64_t count = INDEXED ? a.rows : a.S;  // rows this block's grid walks
-    const int64_t b0 = INDEXED ? 0 : blockIdx.y;
-    if constexpr (!INDEXED) stage_vectors<MODE, kThreads>(a, b0, W8, staged);
+    const int64_t count = a.S;  // rows this block's grid walks
+    const int64_t b = blockIdx.y;
+    stage_vectors<MODE, kThreads>(a, b, W8, staged);
     const U4 *lw = staged, *lk = staged + W8, *lsh = staged + 2 * W8, *lg = staged + 3 * W8;
     const int64_t step = gridDim.x;
     U4 xr[DEPTH][VPT], yr[DEPTH][VPT];
-    int64_t mr[DEPTH];     // INDEXED: the modulation row of each row in the ring
-    int64_t in_lds = -1;   // INDEXED: the modulation row staged in LDS
     // Rows past the end (block-uniform) re-read the last row; only stores are guarded.
-    auto load_row = [&](int64_t i, U4 (&xv)[VPT], U4 (&yv)[VPT], int64_t &m) {
-        const int64_t ic = i < count ? i : count - 1;
-        const int64_t b = INDEXED ? ic / a.S : b0, s = INDEXED ? ic % a.S : ic;
+    auto load_row = [&](int64_t i, U4 (&xv)[VPT], U4 (&yv)[VPT]) {
+        const int64_t s = i < count ? i : count - 1;
 #pragma unroll
         for (int j = 0; j < VPT; ++j) {
             const int c0 = clamp_group(threadIdx.x + j * kThreads, W8) * 8;
             xv[j] = ld16_stream(row_ptr(a.x, b, s) + c0);
             if constexpr (MODE == kGatedRmsModulate) yv[j] = ld16_stream(row_ptr(a.y, b, s) + c0);
         }
-        if constexpr (INDEXED) {
-            int64_t ms;
-            mod_coords(a.index, b, s, m, ms);
-        }
     };
-    auto finish_row = [&](int64_t i, int parity, U4 (&xv)[VPT], U4 (&yv)[VPT], int64_t m) {
+    auto finish_row = [&](int64_t i, int parity, U4 (&xv)[VPT], U4 (&yv)[VPT]) {
         const bool ok = i < count;
-        const int64_t b = INDEXED ? i / a.S : b0, s = INDEXED ? i % a.S : i;
-        if constexpr (INDEXED) {
-            m = uniform64(m);  // every thread loaded the same index
-            if (m != in_lds) {
-                __syncthreads();  // the previous row's reads of the staged vectors are done
-                stage_vectors<MODE, kThreads>(a, m, W8, staged);
-                in_lds = m;
-            }
-        }
+        const int64_t s = i;
         float partial = 0.0f;
 #pragma unroll
         for (int j = 0; j < VPT; ++j) {
@@ -673,18 +650,107 @@ __global__ __launch_bounds__(kThreads) void rms_stream_kernel(RmsArgs a) {
     };
     const int64_t first = blockIdx.x;
 #pragma unroll
-    for (int d = 0; d < DEPTH - 1; ++d) load_row(first + d * step, xr[d], yr[d], mr[d]);
+    for (int d = 0; d < DEPTH - 1; ++d) load_row(first + d * step, xr[d], yr[d]);
     int parity = 0;
     for (int64_t base = first; base < count; base += DEPTH * step) {  // same trip count in every wave
 #pragma unroll
         for (int d = 0; d < DEPTH; ++d) {
             const int64_t i = base + d * step;
             const int nd = (d + DEPTH - 1) % DEPTH;
-            load_row(i + (DEPTH - 1) * step, xr[nd], yr[nd], mr[nd]);
-            finish_row(i, parity, xr[d], yr[d], mr[d]);
+            load_row(i + (DEPTH - 1) * step, xr[nd], yr[nd]);
+            finish_row(i, parity, xr[d], yr[d]);
             parity ^= 1;
         }
     }
+}
+
+// Rows of 64 < W8 <= 256 VPT groups, any modulation rows (broadcast, per row or
+// per token): one row per 256-thread block, thread t owning groups t, t + 256,
+// ... (the fixed order itself). Everything the row needs -- its data, weight and
+// modulation rows (L2 for all but the first blocks) -- is loaded ahead of the
+// arithmetic, so a block is one memory round trip, one reduction and its
+// stores, and the hardware's block scheduler balances the rows. Against the
+// persistent kernels, which stage the vectors in LDS first: RMSNorm + AdaLN at
+// [64, 5376] 3.6 against 10.2 us, [1000, 7168] 9.7 against 14.1 us; the gated op
+// 4.9 against 7.2 us at [256, 5376] and, with per-token rows, 48.4 against 54.9
+// us at [5726, 5376] and 86.8 against 92.8 us at [8192, 7168].
+template <int VPT, int MODE>
+__global__ __launch_bounds__(kThreads) void rms_row_kernel(RmsArgs a) {
+    const uint32_t row = blockIdx.x;  // rows < 2^31
+    const uint32_t b = fast_div(row, a.by_s), s = row - b * static_cast<uint32_t>(a.S);
+    int64_t mb, ms;
+    mod_coords(a.index, b, s, mb, ms);
+    const int W8 = (a.W + 7) / 8;
+    const bf16_t *px = row_ptr(a.x, b, s), *py = row_ptr(a.y, b, s), *pg = row_ptr(a.gate, mb, ms);
+    const bf16_t *psc = row_ptr(a.scale, mb, ms), *psh = row_ptr(a.shift, mb, ms);
+    U4 v[VPT], gv[VPT], yv[VPT], wv[VPT], scv[VPT], shv[VPT];
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+        const int c0 = clamp_group(threadIdx.x + j * kThreads, W8) * 8;
+        v[j] = ld16_stream(px + c0);
+        if constexpr (MODE == kGatedRmsModulate) {
+            yv[j] = ld16_stream(py + c0);
+            gv[j] = ld16(pg + c0);
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+        const int c0 = clamp_group(threadIdx.x + j * kThreads, W8) * 8;
+        wv[j] = ld16(a.w + c0);
+        if constexpr (MODE != kRms) {
+            scv[j] = ld16(psc + c0);
+            shv[j] = ld16(psh + c0);
+        }
+    }
+    __builtin_amdgcn_sched_barrier(0);  // the loads stay together, ahead of the arithmetic
+    float partial = 0.0f;
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+        const int g = threadIdx.x + j * kThreads;
+        v[j] = rms_phase1<MODE>(v[j], gv[j], yv[j], g < W8, partial);
+        if constexpr (MODE == kGatedRmsModulate)
+            if (g < W8) st16_stream(row_ptr_w(a.residual, b, s) + g * 8, v[j]);
+        keep_packed(v[j]);
+    }
+    __shared__ float red[kThreads / 64];
+    const float wsum = fold_lanes<64>(partial);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = wsum;
+    __syncthreads();
+    const float r = rms_reciprocal((red[0] + red[2]) + (red[1] + red[3]), a.W, a.eps_bf);
+#pragma unroll
+    for (int j = 0; j < VPT; ++j) {
+        const int g = threadIdx.x + j * kThreads;
+        const U4 o = rms_phase2<MODE>(v[j], r, wv[j], factor_of(scv[j]), shv[j]);
+        if (g < W8) st16_stream(row_ptr_w(a.out, b, s) + g * 8, o);
+    }
+}
+
+// Where rms_row_kernel is the faster one (16-byte rows, 64 < W8 <= 1024), from
+// graph-timed launches of 64 to 18,000 rows of 1024 to 8192, us, row kernel
+// first:
+//   - rows with their own modulation views (or batches past the grid's y
+//     extent): [300, 5376] 5.8 against 7.4, [8192, 7168] 76.5 against 80.4 (one
+//     row per wave);
+//   - fewer than 1536 rows, which leave the persistent kernels' waves a row each
+//     at most, after the staging: [1000, 5376] 8.4 against 11.2, [1500, 7168]
+//     13.5 against 16.0, [2000, 7168] 16.6 against 17.3, [2000, 5376] 13.5
+//     against 12.9;
+//   - wide rows (W8 > 512) in numbers just above the 2048 that fill the CUs'
+//     first blocks, when part of the CUs run a second one: [3000, 7168] 22.3
+//     against 25.8, [4000, 7168] 28.2 against 26.4;
+//   - the gated op, except over many broadcast rows, where the prefetched rows
+//     of rms_stream_kernel are ahead: [8192, 7168] 86.5 against 86.5,
+//     [18000, 5376] 144 against 141;
+//   - RMSNorm alone, whose one vector is little to load again, at W8 > 512 past
+//     the first 2048 rows: [8192, 7168] 41.3 against 44.7, [2000, 5376] 10.5
+//     against 9.8, [4000, 3072] 11.2 against 9.8.
+template <int MODE>
+bool rows_by_block(const RmsArgs &a, int W8) {
+    if (W8 > 1024) return false;
+    if (a.index.p == nullptr && !a.staged) return true;
+    if (a.rows < 1536 || (W8 > 512 && a.rows > 2048 && a.rows <= 3072)) return true;
+    if (MODE == kGatedRmsModulate) return a.index.p != nullptr || a.rows < 8192;
+    return MODE == kRms && W8 > 512 && a.rows > 2048;
 }
 
 // Rows of W8 > 1024 groups: one row per 256-thread block, VPT groups per
@@ -761,42 +827,41 @@ int launch_rms_vec(const RmsArgs &a, hipStream_t stream) {
         }
         return launch_status();
     }
+    if constexpr (VEC) {
+        if (rows_by_block<MODE>(a, W8)) {
+            const unsigned grid = static_cast<unsigned>(a.rows);
+            switch ((W8 + kThreads - 1) / kThreads) {
+                case 1: rms_row_kernel<1, MODE><<<grid, kThreads, 0, stream>>>(a); break;
+                case 2: rms_row_kernel<2, MODE><<<grid, kThreads, 0, stream>>>(a); break;
+                case 3: rms_row_kernel<3, MODE><<<grid, kThreads, 0, stream>>>(a); break;
+                default: rms_row_kernel<4, MODE><<<grid, kThreads, 0, stream>>>(a); break;
+            }
+            return launch_status();
+        }
+    }
     const int need = (W8 + 63) / 64;
     // Staged vectors: 1 (weight), 3 (+ factor, shift) or 4 (+ gate) rows of W8
     // groups in LDS, within the 64 KiB a workgroup may allocate.
     const int arrays = MODE == kRms ? 1 : (MODE == kRmsModulate ? 3 : 4);
     const size_t lds = static_cast<size_t>(arrays) * W8 * sizeof(U4);
-    if constexpr (VEC && MODE != kRms) {
-        // Per-token modulation rows: rms_stream_kernel over all rows, restaging
-        // the tables' row at each change of index.
-        const int vpt = (W8 + kThreads - 1) / kThreads;
-        if (MODE == kRmsModulate && a.index.p != nullptr && lds <= 65536 && need <= 16) {
+    // EXACT (W8 = 64 G) or the last group partial; G from 2 to 16.
+#define H3_RMS_GROUPS(M) M(2) M(3) M(4) M(5) M(6) M(7) M(8) M(9) M(10) M(11) M(12) M(13) M(14) M(15) M(16)
+    if constexpr (VEC && MODE == kRmsModulate) {
+        if (a.index.p != nullptr && lds <= 65536 && need <= 16) {
             constexpr int kWaves = kStagedThreads / 64;
             const int64_t groups = (a.rows + kWaves - 1) / kWaves;
-            const bool exact = W8 % 64 == 0;
             const unsigned grid = static_cast<unsigned>(groups < kStagedBlocks ? groups : kStagedBlocks);
-#define H3_RMS_MOD_INDEXED(GG)                                                                                    \
-    if (need <= GG) {                                                                                            \
-        if (exact && W8 == 64 * GG)                                                                              \
-            rms_modulate_indexed_kernel<GG, kStagedThreads, true><<<grid, kStagedThreads, lds, stream>>>(a);    \
-        else                                                                                                     \
-            rms_modulate_indexed_kernel<GG, kStagedThreads, false><<<grid, kStagedThreads, lds, stream>>>(a);   \
-        return launch_status();                                                                                  \
-    }
-            H3_RMS_MOD_INDEXED(2) H3_RMS_MOD_INDEXED(3) H3_RMS_MOD_INDEXED(4) H3_RMS_MOD_INDEXED(6)
-            H3_RMS_MOD_INDEXED(8) H3_RMS_MOD_INDEXED(10) H3_RMS_MOD_INDEXED(12) H3_RMS_MOD_INDEXED(14)
-            H3_RMS_MOD_INDEXED(16)
+            switch (need) {
+#define H3_RMS_MOD_INDEXED(GG)                                                                                  \
+    case GG:                                                                                                   \
+        if (W8 % 64 == 0)                                                                                      \
+            rms_modulate_indexed_kernel<GG, kStagedThreads, true><<<grid, kStagedThreads, lds, stream>>>(a);  \
+        else                                                                                                   \
+            rms_modulate_indexed_kernel<GG, kStagedThreads, false><<<grid, kStagedThreads, lds, stream>>>(a); \
+        return launch_status();
+                H3_RMS_GROUPS(H3_RMS_MOD_INDEXED)
 #undef H3_RMS_MOD_INDEXED
-        }
-        if (a.index.p != nullptr && lds <= 65536 && vpt <= 4) {
-            const unsigned grid = static_cast<unsigned>(a.rows < kStreamBlocks ? a.rows : kStreamBlocks);
-#define H3_RMS_STREAM_INDEXED(V)                                                            \
-    if (vpt <= V) {                                                                        \
-        rms_stream_kernel<V, MODE, kStreamDepth, true><<<grid, kThreads, lds, stream>>>(a); \
-        return launch_status();                                                            \
-    }
-            H3_RMS_STREAM_INDEXED(1) H3_RMS_STREAM_INDEXED(2) H3_RMS_STREAM_INDEXED(3) H3_RMS_STREAM_INDEXED(4)
-#undef H3_RMS_STREAM_INDEXED
+            }
         }
     }
     if (VEC && a.staged && lds <= 65536) {
@@ -808,39 +873,43 @@ int launch_rms_vec(const RmsArgs &a, hipStream_t stream) {
                 const int vpt = (W8 + kThreads - 1) / kThreads;
 #define H3_RMS_STREAM(V)                                                                    \
     if (vpt <= V) {                                                                        \
-        rms_stream_kernel<V, MODE, kStreamDepth, false><<<grid, kThreads, lds, stream>>>(a); \
+        rms_stream_kernel<V, MODE, kStreamDepth><<<grid, kThreads, lds, stream>>>(a); \
         return launch_status();                                                            \
     }
                 H3_RMS_STREAM(1) H3_RMS_STREAM(2) H3_RMS_STREAM(3) H3_RMS_STREAM(4)
 #undef H3_RMS_STREAM
             } else if (need <= 16) {
                 constexpr int kWaves = kStagedThreads / 64;
-                // EXACT (W8 = 64 G): three blocks per CU; otherwise about two.
-                const bool exact = W8 % 64 == 0;
-                int cus = exact ? stream_device_cus(stream) : 0;
-                const int64_t blocks = exact && cus > 0 ? 3 * static_cast<int64_t>(cus) : kStagedBlocks;
+                const int cus = stream_device_cus(stream);
+                // Three blocks per CU from 32 rows per CU on, two below, where a
+                // third one's waves get no second row to overlap with their
+                // staging: 46.1 against 48.9 us at [8192, 7168] and 74.4 against
+                // 76.8 us at [18000, 5376], but 36.6 against 34.5 us at
+                // [5726, 7168] and 29.0 against 27.7 us at [5726, 5376].
+                const int64_t blocks = cus > 0 ? (a.rows >= 32 * static_cast<int64_t>(cus) ? 3 : 2) * static_cast<int64_t>(cus)
+                                               : kStagedBlocks;
                 const int64_t per_entry = (blocks + batch - 1) / batch;
                 const int64_t needed = (a.S + kWaves - 1) / kWaves;
                 const dim3 grid(static_cast<unsigned>(needed < per_entry ? needed : per_entry), batch);
+                switch (need) {
 #define H3_RMS_STAGED(GG)                                                                               \
-    if (need <= GG) {                                                                                  \
-        if (exact && W8 == 64 * GG)                                                                    \
+    case GG:                                                                                           \
+        if (W8 % 64 == 0)                                                                              \
             rms_staged_kernel<GG, MODE, kStagedThreads, true><<<grid, kStagedThreads, lds, stream>>>(a);  \
         else                                                                                           \
             rms_staged_kernel<GG, MODE, kStagedThreads, false><<<grid, kStagedThreads, lds, stream>>>(a); \
-        return launch_status();                                                                        \
-    }
-                H3_RMS_STAGED(2) H3_RMS_STAGED(3) H3_RMS_STAGED(4) H3_RMS_STAGED(6) H3_RMS_STAGED(8)
-                H3_RMS_STAGED(10) H3_RMS_STAGED(12) H3_RMS_STAGED(14) H3_RMS_STAGED(16)
+        return launch_status();
+                    H3_RMS_GROUPS(H3_RMS_STAGED)
 #undef H3_RMS_STAGED
+                }
             }
         }
     }
-    if (need <= 16) {
+    if (!VEC && need <= 16) {
         const unsigned grid = static_cast<unsigned>((a.rows + kThreads / 64 - 1) / (kThreads / 64));
 #define H3_RMS_WAVE(GG)                                                            \
     if (need <= GG) {                                                             \
-        rms_wave_kernel<GG, VEC, MODE><<<grid, kThreads, 0, stream>>>(a);         \
+        rms_wave_kernel<GG, MODE><<<grid, kThreads, 0, stream>>>(a);              \
         return launch_status();                                                   \
     }
         H3_RMS_WAVE(2) H3_RMS_WAVE(3) H3_RMS_WAVE(4) H3_RMS_WAVE(6) H3_RMS_WAVE(8) H3_RMS_WAVE(10)

@@ -1,0 +1,67 @@
+"""The RMS family's 16-byte launch shapes at the sizes where the rule that picks
+them changes (rows_by_block) and at the edges of their groups: bitwise against
+the oracle's fixed order, on rows taken from every part of the launch."""
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+BF = torch.bfloat16
+EPS = 1e-6
+
+
+def _randn(gen, *shape, scale=1.0, mean=0.0):
+    return (torch.randn(*shape, generator=gen) * scale + mean).to(BF)
+
+
+# One launch per side of every bound: 1536 rows, 2048 / 3072 rows of W8 > 512,
+# 8192 gated rows; W8 = 65 (one group past a wave), 512 / 513, 672 (a half last
+# wave group), 768 and 1024 (exact), 1023.
+@pytest.mark.parametrize("rows,W", [
+    (1535, 520), (1536, 520), (1536, 4096), (1537, 4104), (2048, 5376), (2049, 5376), (3072, 8184), (3073, 8192),
+    (1600, 6144), (8191, 5376), (8192, 5376),
+])
+@pytest.mark.parametrize("mods", ["broadcast", "per_token", "per_row"])
+def test_rms_family_launch_shapes_bitwise(pkg, oracle, device, rows, W, mods):
+    if mods == "per_row" and rows not in (1537, 2049):
+        pytest.skip("per-row views take one launch shape")
+    gen = torch.Generator("cpu").manual_seed(rows + W)
+    R = 3
+    B, S = (3, rows // 3) if rows % 3 == 0 else (1, rows)
+    x, y = _randn(gen, B, S, W), _randn(gen, B, S, W)
+    w = _randn(gen, W, scale=0.1, mean=1.0)
+    tables = [_randn(gen, R, W, scale=0.1) for _ in range(3)]
+    # Runs of rows, one boundary inside a block of eight rows.
+    index = (torch.arange(B * S) * R // (B * S)).view(B, S)
+    if mods == "broadcast":
+        index = torch.zeros(B, S, dtype=torch.int64)
+    gate, scale, shift = (t[index] for t in tables)  # [B, S, W]
+    d = lambda t: t.to(device)
+    xd, yd, wd = d(x), d(y), d(w)
+    outs = [torch.full((B, S, W), float("nan"), dtype=BF, device=device) for _ in range(4)]
+    mod, res, norm, plain = outs
+    if mods == "per_token":
+        gt, sc, sh = (d(t) for t in tables)
+        pkg.make_rms_modulate_indexed()(xd, wd, EPS, sc, sh, d(index), mod)
+        pkg.make_gated_residual_rms_modulate_indexed()(xd, gt, yd, wd, EPS, sc, sh, d(index), res, norm)
+    else:
+        views = [d(t) for t in (gate, scale, shift)]
+        if mods == "broadcast":
+            views = [d(t)[:1].unsqueeze(0).expand(B, S, W) for t in tables]
+        gt, sc, sh = views
+        pkg.make_rms_modulate()(xd, wd, EPS, sc, sh, mod)
+        pkg.make_gated_residual_rms_modulate()(xd, gt, yd, wd, EPS, sc, sh, res, norm)
+    pkg.make_rms(width=None)(xd, wd, EPS, plain)
+    torch.cuda.synchronize()
+    for t in outs:
+        assert not torch.isnan(t).any()
+    rows_at = torch.unique(torch.cat([torch.arange(9), torch.arange(S - 9, S), S // R + torch.arange(-9, 9),
+                                      torch.randint(0, S, (32,), generator=gen)]).clamp(0, S - 1))
+    pick = lambda t: t[:, rows_at].contiguous()
+    want_res, want_norm = oracle.gated_residual_rms_modulate(pick(x), pick(gate), pick(y), w, EPS, pick(scale),
+                                                             pick(shift))
+    want = {"mod": oracle.rms_modulate(pick(x), w, EPS, pick(scale), pick(shift)), "res": want_res,
+            "norm": want_norm, "plain": oracle.rms_norm(pick(x), w, EPS)}
+    for name, got in zip(("mod", "res", "norm", "plain"), outs):
+        assert torch.equal(pick(got.cpu()), want[name]), name
