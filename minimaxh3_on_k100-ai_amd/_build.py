@@ -1,5 +1,6 @@
 """Build recipe for libh3mi355x.so: every csrc/*.hip compiled for gfx950 with
-hipcc, linked into one shared library next to this file.
+hipcc, linked into one shared library next to this file; and for _h3call.so, the
+Python face's native call into it (csrc/h3_call.cpp, host code only).
 
     python -m <package>._build        (or __graft_entry__.build())
 """
@@ -16,6 +17,7 @@ PACKAGE_DIR = Path(__file__).resolve().parent
 CSRC = PACKAGE_DIR / "csrc"
 BUILD_DIR = PACKAGE_DIR / "_build"
 LIBRARY = PACKAGE_DIR / "libh3mi355x.so"
+CALL_MODULE = PACKAGE_DIR / "_h3call.so"
 ARCH = "gfx950"
 
 # -packed-fp32-ops: keep hipcc from forming v_pk_{add,mul,fma}_f32 (some of
@@ -47,14 +49,37 @@ def _compile(source: Path) -> Path:
     return obj
 
 
+def _build_call_module() -> Path:
+    """The host-only CPython module, against torch's headers and libraries."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+
+    tmp = CALL_MODULE.with_suffix(".so.tmp")
+    lib_dir = Path(torch.__file__).resolve().parent / "lib"
+    cmd = [os.environ.get("CXX") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           *(f"-isystem{p}" for p in cpp_extension.include_paths()), f"-isystem{sysconfig.get_paths()['include']}",
+           str(CSRC / "h3_call.cpp"), f"-L{lib_dir}", "-lc10", "-ltorch_cpu", "-ltorch_python",
+           f"-Wl,-rpath,{lib_dir}", "-o", str(tmp)]
+    proc = subprocess.run(cmd, capture_output=True, text=True)
+    if proc.returncode != 0:
+        raise RuntimeError(f"building {CALL_MODULE.name} failed:\n{proc.stderr}")
+    os.replace(tmp, CALL_MODULE)
+    return CALL_MODULE
+
+
 def build(verbose: bool = True) -> Path:
-    """Compile every HIP source and link libh3mi355x.so (always rebuilds)."""
+    """Compile every HIP source and link libh3mi355x.so and _h3call.so (always rebuilds)."""
     sources = sorted(CSRC.glob("*.hip"))
     if not sources:
         raise RuntimeError(f"no HIP sources under {CSRC}")
     BUILD_DIR.mkdir(exist_ok=True)
-    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(sources))) as pool:
+    with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, len(sources) + 1)) as pool:
+        call_module = pool.submit(_build_call_module)
         objects = list(pool.map(_compile, sources))
+        call_module.result()
     tmp = LIBRARY.with_suffix(".so.tmp")
     cmd = [hipcc(), f"--offload-arch={ARCH}", "-shared", "-fPIC", *map(str, objects), "-o", str(tmp)]
     proc = subprocess.run(cmd, capture_output=True, text=True)
@@ -62,7 +87,7 @@ def build(verbose: bool = True) -> Path:
         raise RuntimeError(f"link failed:\n{proc.stderr}")
     os.replace(tmp, LIBRARY)
     if verbose:
-        print(f"built {LIBRARY} from {len(sources)} sources")
+        print(f"built {LIBRARY} from {len(sources)} sources and {CALL_MODULE.name}")
     return LIBRARY
 
 

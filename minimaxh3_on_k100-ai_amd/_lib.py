@@ -5,10 +5,16 @@ element strides, scalars as {&double, NULL, NULL}, and every launch goes to the
 current torch stream of the tensors' device, mirroring how the reference's
 InfiniCore launchers fill the struct (patches/InfiniCore.patch:1062-1089).
 There is no fallback: a missing library or a non-zero status raises.
+
+`fast` binds an entry point through the native module _h3call (csrc/h3_call.cpp)
+for the plain case of a call; the factories try it first and take the checked
+ctypes path below for everything else.
 """
 from __future__ import annotations
 
 import ctypes
+import functools
+import importlib
 from pathlib import Path
 from typing import Sequence
 
@@ -108,6 +114,34 @@ def entry(name: str):
     return fn
 
 
+_fast_calls: dict = {}  # the bound calls, one per distinct argument list of `fast`
+
+
+def _not_taken(*args) -> bool:
+    return False
+
+
+def fast(name: str, kinds: str, order: tuple | None = None, fix: tuple | None = None):
+    """A callable that launches entry point `name` when every argument is as
+    `kinds` says (csrc/h3_call.cpp: a kind and a rank per argument) and returns
+    whether it did. order: the launcher's arguments by index of the call's;
+    fix: (argument, dim, size) that must hold. Without the library it takes no
+    call, and the ctypes path raises at first use."""
+    key = (name, kinds, order, fix)
+    bound = _fast_calls.get(key)
+    if bound is None:
+        if not LIBRARY_PATH.exists():
+            return _not_taken
+        try:
+            native = importlib.import_module(__package__ + "._h3call")
+        except ImportError as e:
+            raise ImportError("_h3call.so is missing or does not load: build it with __graft_entry__.build()") from e
+        address = ctypes.cast(getattr(library(), name), ctypes.c_void_p).value
+        order = tuple(range(len(kinds) // 2)) if order is None else order
+        bound = _fast_calls[key] = functools.partial(native.call, native.plan(address, kinds, order, fix))
+    return bound
+
+
 def _workspace_query(name: str, *sizes: int) -> int:
     fn = _bound.get(name)
     if fn is None:
@@ -124,6 +158,13 @@ def _workspace_query(name: str, *sizes: int) -> int:
 def attention_workspace_bytes(B: int, H: int, Sq: int, Sk: int) -> int:
     """h3_full_attention_workspace_bytes on the current device (0: no split)."""
     return _workspace_query("h3_full_attention_workspace_bytes", B, H, Sq, Sk)
+
+
+@functools.lru_cache(maxsize=4096)
+def planned_workspace(device_index: int, B: int, H: int, Sq: int, Sk: int, head_dim: int) -> int:
+    """attention_planned_workspace_bytes on a device, kept by its sizes."""
+    with torch.cuda.device(device_index):
+        return attention_planned_workspace_bytes(B, H, Sq, Sk, head_dim)
 
 
 def attention_planned_workspace_bytes(B: int, H: int, Sq: int, Sk: int, head_dim: int) -> int:

@@ -33,6 +33,8 @@ and `make_attention_fp8pv` (bf16 logits, fp8 P.V).
 """
 from __future__ import annotations
 
+import functools
+
 import torch
 
 from . import _lib
@@ -79,28 +81,51 @@ def make_attention(block_m=128, block_n=32, num_warps=4, num_stages=1, caller="t
         entry = "launch_h3_full_attention_bf16_prescale" if numerics == "bf16_prescale" else "launch_h3_full_attention"
 
     split = split_last_round and numerics != "bf16_prescale"
-    plans: dict = {}  # (device, B, H, Sq, Sk) -> workspace bytes
+    if split:
+        fast = _lib.fast("launch_h3_attention_planned", "b4b4b4s0b4w1", fix=(0, 3, head_dim))
+    else:
+        fast = _lib.fast(entry, "b4b4b4s0b4", fix=(0, 3, head_dim))
 
-    def kernel(q, k, v, scale, out):
+    def check(q, k, v, out):
         _check_qkvo(q, k, v, out)
         if q.shape[3] != head_dim:
             raise ValueError(f"this kernel is built for head_dim {head_dim}, got tensors of head dim {q.shape[3]}")
         device = _lib.check_cuda(q, k, v, out)
         _lib.check_dtype(torch.bfloat16, q, k, v, out)
-        if split:
-            key = (device, q.shape[0], q.shape[1], q.shape[2], k.shape[2])
-            nbytes = plans.get(key)
-            if nbytes is None:
-                with torch.cuda.device(device):
-                    nbytes = plans[key] = _lib.attention_planned_workspace_bytes(*key[1:], head_dim)
-            ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
-            _lib.launch("launch_h3_attention_planned", device, _lib.tensor(q), _lib.tensor(k), _lib.tensor(v),
-                        _lib.scalar(scale), _lib.tensor(out), _lib.tensor(ws))
+        return device
+
+    if not split:
+        def kernel(q, k, v, scale, out):
+            if fast(q, k, v, scale, out):
+                return
+            _lib.launch(entry, check(q, k, v, out), _lib.tensor(q), _lib.tensor(k), _lib.tensor(v),
+                        _lib.scalar(scale), _lib.tensor(out))
+
+        return kernel
+
+    workspaces: dict = {}  # (q shape, k shape, device index) -> workspace bytes
+
+    def kernel(q, k, v, scale, out):
+        key = (q.shape, k.shape, q.get_device())
+        nbytes = workspaces.get(key)
+        if nbytes is None:
+            device = check(q, k, v, out)
+            nbytes = workspaces[key] = _lib.planned_workspace(device.index, *q.shape[:3], k.shape[2], head_dim)
+        ws = None if nbytes == 0 else torch.empty(nbytes, dtype=torch.uint8, device=q.device)
+        if fast(q, k, v, scale, out, ws):
             return
-        _lib.launch(entry, device, _lib.tensor(q), _lib.tensor(k), _lib.tensor(v), _lib.scalar(scale),
-                    _lib.tensor(out))
+        device = check(q, k, v, out)
+        if ws is None:
+            ws = torch.empty(0, dtype=torch.uint8, device=device)
+        _lib.launch("launch_h3_attention_planned", device, _lib.tensor(q), _lib.tensor(k), _lib.tensor(v),
+                    _lib.scalar(scale), _lib.tensor(out), _lib.tensor(ws))
 
     return kernel
+
+
+@functools.lru_cache(maxsize=None)
+def _slots_fast():
+    return _lib.fast("launch_h3_quantize_fp8_per_head_slots", "b4c2e4c1")
 
 
 def quantize_fp8_per_head(x: torch.Tensor, transposed: bool = False, x8: torch.Tensor | None = None,
@@ -113,6 +138,8 @@ def quantize_fp8_per_head(x: torch.Tensor, transposed: bool = False, x8: torch.T
     amax_slots: fp32 [H, 64] per-head maxima of |x| already folded by the
     producer (make_qkv_norm_rope_pack_fp8_vamax); then only the code pass
     reads x."""
+    if amax_slots is not None and x8 is not None and descale is not None and _slots_fast()(x, amax_slots, x8, descale):
+        return x8, descale
     if x.dim() != 4:
         raise ValueError("x must be [B, H, S, D]")
     device = _lib.check_cuda(x)
@@ -156,8 +183,11 @@ def make_attention_fp8():
     e4m3 per 64-key tile). v8 must be S-contiguous (quantize_fp8_per_head(v,
     transposed=True)). Returns kernel(q8, k8, v8, q_descale, k_descale,
     v_descale, scale, out) with out bf16 [B, H, Sq, 128]."""
+    fast = _lib.fast("launch_h3_full_attention_fp8", "e4e4e4c1c1c1s0b4")
 
     def kernel(q8, k8, v8, q_descale, k_descale, v_descale, scale, out):
+        if fast(q8, k8, v8, q_descale, k_descale, v_descale, scale, out):
+            return
         _check_qkvo(q8, k8, v8, out)
         device = _lib.check_cuda(q8, k8, v8, q_descale, k_descale, v_descale, out)
         _lib.check_dtype(torch.float8_e4m3fn, q8, k8, v8)
@@ -204,8 +234,11 @@ def make_attention_fp8x2():
     fp32 sum of the unquantised P (make_attention_fp8 sums the quantised one).
     Returns kernel(q8, q8_lo, k8, k8_lo, v8, q_descale, k_descale, v_descale,
     scale, out). No counterpart in the reference."""
+    fast = _lib.fast("launch_h3_full_attention_fp8x2", "e4e4e4e4e4c1c1c1s0b4")
 
     def kernel(q8, q8_lo, k8, k8_lo, v8, q_descale, k_descale, v_descale, scale, out):
+        if fast(q8, q8_lo, k8, k8_lo, v8, q_descale, k_descale, v_descale, scale, out):
+            return
         _check_qkvo(q8, k8, v8, out)
         if q8_lo.shape != q8.shape or k8_lo.shape != k8.shape:
             raise ValueError("the lo codes must match the hi codes' shapes")
@@ -225,8 +258,11 @@ def make_attention_fp8pv():
     """bf16 logits with an fp8 P.V product: q, k bf16 as for make_attention;
     v8 e4m3fn S-contiguous with v_descale. Returns kernel(q, k, v8, v_descale,
     scale, out)."""
+    fast = _lib.fast("launch_h3_full_attention_fp8pv", "b4b4e4c1s0b4")
 
     def kernel(q, k, v8, v_descale, scale, out):
+        if fast(q, k, v8, v_descale, scale, out):
+            return
         _check_qkvo(q, k, v8, out)
         device = _lib.check_cuda(q, k, v8, v_descale, out)
         _lib.check_dtype(torch.bfloat16, q, k, out)

@@ -49,8 +49,11 @@ def _ndim(n: int, **tensors: torch.Tensor) -> None:
 def make_swiglu(caller="torch", output_dir=None, archs=None, rows=1, cols=1024, num_warps=4, dtype=None):
     """out = bf16(up * bf16(g / (1 + exp(-g)))) on [B, S, F] (tools/h3_pointwise.py:18-34)."""
     _bf16_only(dtype)
+    fast = _lib.fast("launch_h3_swiglu_exact", "b3b3b3")
 
     def kernel(up, gate, out):
+        if fast(up, gate, out):
+            return
         _ndim(3, up=up, gate=gate, out=out)
         device = _bf16(up, gate, out)
         _lib.launch("launch_h3_swiglu_exact", device, _lib.tensor(up), _lib.tensor(gate), _lib.tensor(out))
@@ -64,8 +67,11 @@ def make_rms(caller="torch", output_dir=None, archs=None, width=5376, dtype=None
     if width is not None and width <= 0:
         raise ValueError("width must be positive")
     name = {128: "launch_h3_rms_exact_128", 5376: "launch_h3_rms_exact_5376"}.get(width, "launch_h3_rms_exact")
+    fast = _lib.fast(name, "b3b1s0b3", fix=None if width is None else (0, 2, width))
 
     def kernel(x, weight, eps, out):
+        if fast(x, weight, eps, out):
+            return
         _ndim(3, x=x, out=out)
         _ndim(1, weight=weight)
         if width is not None and x.shape[-1] != width:
@@ -80,8 +86,11 @@ def make_rms_modulate(caller="torch", output_dir=None, archs=None, dtype=None):
     """RMSNorm + AdaLN: bf16(bf16(bf16(rms(x) w) bf16(1 + scale)) + shift)
     (tools/h3_pointwise.py:83-108), any width."""
     _bf16_only(dtype)
+    fast = _lib.fast("launch_h3_rms_modulate_exact", "b3b1s0b3b3b3")
 
     def kernel(x, weight, eps, scale, shift, out):
+        if fast(x, weight, eps, scale, shift, out):
+            return
         _ndim(3, x=x, scale=scale, shift=shift, out=out)
         _ndim(1, weight=weight)
         device = _bf16(x, weight, scale, shift, out)
@@ -94,8 +103,11 @@ def make_rms_modulate(caller="torch", output_dir=None, archs=None, dtype=None):
 def make_gated_residual(caller="torch", output_dir=None, archs=None, block=(4, 512), num_warps=8, dtype=None):
     """out = bf16(x + bf16(gate * y)) (tools/h3_pointwise.py:121-136)."""
     _bf16_only(dtype)
+    fast = _lib.fast("launch_h3_gated_residual_exact", "b3b3b3b3")
 
     def kernel(x, gate, y, out):
+        if fast(x, gate, y, out):
+            return
         _ndim(3, x=x, gate=gate, y=y, out=out)
         device = _bf16(x, gate, y, out)
         _lib.launch("launch_h3_gated_residual_exact", device, _lib.tensor(x), _lib.tensor(gate),
@@ -108,8 +120,11 @@ def make_gated_residual_rms_modulate(caller="torch", output_dir=None, archs=None
     """residual = bf16(x + bf16(gate * y)); out = rms_modulate(residual)
     (tools/h3_pointwise.py:150-182)."""
     _bf16_only(dtype)
+    fast = _lib.fast("launch_h3_gated_residual_rms_modulate_exact", "b3b3b3b1s0b3b3b3b3")
 
     def kernel(x, gate, y, weight, eps, scale, shift, residual, out):
+        if fast(x, gate, y, weight, eps, scale, shift, residual, out):
+            return
         _ndim(3, x=x, gate=gate, y=y, scale=scale, shift=shift, residual=residual, out=out)
         _ndim(1, weight=weight)
         device = _bf16(x, gate, y, weight, scale, shift, residual, out)
@@ -170,8 +185,11 @@ def make_rms_modulate_indexed(check_indices: bool = True):
     kernel(x, weight, eps, scale, shift, index, out). check_indices=False skips
     the range check (no host synchronisation; out-of-range indices are clamped
     by the kernel)."""
+    fast = _lib.fast("launch_h3_rms_modulate_indexed", "b3b1s0b2b2i2b3")
 
     def kernel(x, weight, eps, scale, shift, index, out):
+        if not check_indices and fast(x, weight, eps, scale, shift, index, out):
+            return
         _ndim(3, x=x, out=out)
         _ndim(2, scale=scale, shift=shift)
         _ndim(1, weight=weight)
@@ -188,8 +206,11 @@ def make_gated_residual_rms_modulate_indexed(check_indices: bool = True):
     """residual = bf16(x + bf16(gate * y)); out = rms_modulate(residual), with
     gate/scale/shift rows index[b, s] of [R, W] tables. Returns
     kernel(x, gate, y, weight, eps, scale, shift, index, residual, out)."""
+    fast = _lib.fast("launch_h3_gated_residual_rms_modulate_indexed", "b3b2b3b1s0b2b2i2b3b3")
 
     def kernel(x, gate, y, weight, eps, scale, shift, index, residual, out):
+        if not check_indices and fast(x, gate, y, weight, eps, scale, shift, index, residual, out):
+            return
         _ndim(3, x=x, y=y, residual=residual, out=out)
         _ndim(2, gate=gate, scale=scale, shift=shift)
         _ndim(1, weight=weight)
@@ -205,8 +226,11 @@ def make_gated_residual_rms_modulate_indexed(check_indices: bool = True):
 def make_gated_residual_indexed(check_indices: bool = True):
     """out = bf16(x + bf16(gate * y)) with the gate row index[b, s] of a [R, W]
     table. Returns kernel(x, gate, y, index, out)."""
+    fast = _lib.fast("launch_h3_gated_residual_indexed", "b3b2b3i2b3")
 
     def kernel(x, gate, y, index, out):
+        if not check_indices and fast(x, gate, y, index, out):
+            return
         _ndim(3, x=x, y=y, out=out)
         _ndim(2, gate=gate)
         device = _bf16(x, gate, y, out)
@@ -221,8 +245,11 @@ def make_rope(caller="torch", output_dir=None, archs=None, dtype=None):
     """Rotate-half RoPE on channels 0..95 of [S, H, 128], cos/sin [S, 48]
     (tools/h3_pointwise.py:199-231). Returns launch(x, cos, sin, out)."""
     _bf16_only(dtype)
+    fast = _lib.fast("launch_h3_rope_exact", "b3b2b2b3", (0, 0, 0, 1, 2, 3, 3, 3))
 
     def launch(x, cos, sin, out):
+        if fast(x, cos, sin, out):
+            return
         _ndim(3, x=x, out=out)
         _ndim(2, cos=cos, sin=sin)
         device = _bf16(x, cos, sin, out)
@@ -254,8 +281,11 @@ def make_qk_norm_rope(caller="torch", output_dir=None, archs=None, rows=8, num_w
         raise ValueError("qk_norm_rope: block_tokens > 1 needs ranks == 1")
     if caller != "torch":
         return _qk_raw
+    fast = _lib.fast("launch_h3_qk_norm_rope", "b4b1s0b2b2b4", (0, 0, 0, 1, 1, 1, 2, 3, 4, 5, 5, 5))
 
     def launch(x, weight, eps, cos, sin, out):
+        if fast(x, weight, eps, cos, sin, out):
+            return
         _qk_raw(x, x, x, weight, weight, weight, eps, cos, sin, out, out, out)
 
     return launch
@@ -286,8 +316,11 @@ def make_qkv_norm_rope_pack(dtype=None):
     the outputs are typically send buffers [P, T, Hs, 128] permuted to
     [T, P, Hs, 128]); positions int64 [T] (int32 is widened)."""
     _bf16_only(dtype)
+    fast = _lib.fast("launch_h3_qkv_norm_rope_pack", "b4b4b4b1b1s0t2l1b4b4b4")
 
     def kernel(q, k, v, q_weight, k_weight, eps, cache, positions, q_out, k_out, v_out):
+        if fast(q, k, v, q_weight, k_weight, eps, cache, positions, q_out, k_out, v_out):
+            return
         _ndim(4, q=q, k=k, v=v, q_out=q_out, k_out=k_out, v_out=v_out)
         _ndim(1, q_weight=q_weight, k_weight=k_weight, positions=positions)
         _ndim(2, cache=cache)
@@ -322,9 +355,13 @@ def make_qkv_norm_rope_pack_fp8(dtype=None):
     [P * Hs] receive bound / 448; v_out bf16 (quantise it with
     quantize_fp8_per_head). No counterpart in the reference."""
     _bf16_only(dtype)
+    fast = _lib.fast("launch_h3_qkv_norm_rope_pack_fp8", "b4b4b4b1b1s0t2l1u4u4b4f1f1")
 
     def kernel(q, k, v, q_weight, k_weight, eps, cache, positions, q8, k8, v_out, q_descale, k_descale,
                _entry="launch_h3_qkv_norm_rope_pack_fp8", _extra=()):
+        if not _extra and fast(q, k, v, q_weight, k_weight, eps, cache, positions, q8, k8, v_out, q_descale,
+                               k_descale):
+            return
         _ndim(4, q=q, k=k, v=v, q8=q8, k8=k8, v_out=v_out)
         _ndim(1, q_weight=q_weight, k_weight=k_weight, positions=positions, q_descale=q_descale,
               k_descale=k_descale)
@@ -357,8 +394,11 @@ def make_qkv_norm_rope_pack_fp8_vamax(dtype=None):
     extends is patches/InfiniLM.patch:1063-1069,1104."""
     _bf16_only(dtype)
     base = make_qkv_norm_rope_pack_fp8()
+    fast = _lib.fast("launch_h3_qkv_norm_rope_pack_fp8_vamax", "b4b4b4b1b1s0t2l1u4u4b4f1f1c2")
 
     def kernel(q, k, v, q_weight, k_weight, eps, cache, positions, q8, k8, v_out, q_descale, k_descale, v_amax):
+        if fast(q, k, v, q_weight, k_weight, eps, cache, positions, q8, k8, v_out, q_descale, k_descale, v_amax):
+            return
         _ndim(2, v_amax=v_amax)
         _lib.check_cuda(q, v_amax)
         _lib.check_dtype(torch.float32, v_amax)
@@ -379,9 +419,13 @@ def make_qkv_norm_rope_pack_fp8x2_vamax(dtype=None):
     e4m3fn (or uint8) with the shapes and strides of q8, k8. No counterpart in
     the reference."""
     _bf16_only(dtype)
+    fast = _lib.fast("launch_h3_qkv_norm_rope_pack_fp8x2_vamax", "b4b4b4b1b1s0t2l1u4u4u4u4b4f1f1c2")
 
     def kernel(q, k, v, q_weight, k_weight, eps, cache, positions, q8, q8_lo, k8, k8_lo, v_out, q_descale,
                k_descale, v_amax):
+        if fast(q, k, v, q_weight, k_weight, eps, cache, positions, q8, q8_lo, k8, k8_lo, v_out, q_descale,
+                k_descale, v_amax):
+            return
         _ndim(4, q8_lo=q8_lo, k8_lo=k8_lo)
         _ndim(2, v_amax=v_amax)
         _lib.check_cuda(q, q8_lo, k8_lo, v_amax)
@@ -462,8 +506,11 @@ def make_qk_norm_rope_interleaved(dtype=None):
     Returns launch(x, weight, eps, cos, sin, out). No counterpart in the
     reference; it serves the 32/48/48 interleaved RoPE layout."""
     _bf16_only(dtype)
+    fast = _lib.fast("launch_h3_qk_norm_rope_interleaved", "b4b1s0b2b2b4")
 
     def launch(x, weight, eps, cos, sin, out):
+        if fast(x, weight, eps, cos, sin, out):
+            return
         _ndim(4, x=x, out=out)
         _ndim(1, weight=weight)
         _ndim(2, cos=cos, sin=sin)
@@ -480,8 +527,11 @@ def make_qk_norm_rope_interleaved_qk(dtype=None):
     launch(q, k, q_weight, k_weight, eps, cos, sin, q_out, k_out), bitwise equal
     to the two single-tensor launches. No counterpart in the reference."""
     _bf16_only(dtype)
+    fast = _lib.fast("launch_h3_qk_norm_rope_interleaved_qk", "b4b4b1b1s0b2b2b4b4")
 
     def launch(q, k, q_weight, k_weight, eps, cos, sin, q_out, k_out):
+        if fast(q, k, q_weight, k_weight, eps, cos, sin, q_out, k_out):
+            return
         _ndim(4, q=q, k=k, q_out=q_out, k_out=k_out)
         _ndim(1, q_weight=q_weight, k_weight=k_weight)
         _ndim(2, cos=cos, sin=sin)
@@ -498,8 +548,11 @@ def make_rope_cache(caller="torch", output_dir=None, archs=None, block_tokens=64
     [T, 48] bf16 views (tools/h3_pointwise.py:405-442).
     Returns kernel(position, power, cos, sin)."""
     _bf16_only(dtype)
+    fast = _lib.fast("launch_h3_rope_cache", "d2f1b2b2")
 
     def kernel(position, power, cos, sin):
+        if fast(position, power, cos, sin):
+            return
         _ndim(2, position=position, cos=cos, sin=sin)
         _ndim(1, power=power)
         device = _lib.check_cuda(position, power, cos, sin)

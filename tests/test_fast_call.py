@@ -1,0 +1,110 @@
+"""The native call path of the factories (csrc/h3_call.cpp): what it takes and
+what it leaves to the checked Python path."""
+from __future__ import annotations
+
+import importlib
+
+import pytest
+import torch
+
+BF = torch.bfloat16
+EPS = 1e-6
+
+
+@pytest.fixture()
+def native():
+    return importlib.import_module("minimaxh3_on_k100-ai_amd._h3call")
+
+
+def test_plan_arguments_are_checked(native):
+    for args in [(0, "", (), None), (0, "b3", (1,), None), (0, "b3", [0], None), (0, "b3", (0,), (1, 0, 5)),
+                 (0, "b3", (0,), (0, 3, 5)), (0, "b3" * 17, (0,), None), (0, "t2" * 11, tuple(range(11)), None)]:
+        with pytest.raises((ValueError, TypeError)):
+            native.plan(*args)
+    with pytest.raises(ValueError):
+        native.call(object(), 1)
+
+
+def test_other_than_plain_cuda_tensors_are_not_taken(native):
+    """No address is called: wrong counts, types and devices return False
+    before the launch."""
+    plan = native.plan(0, "b3b1s0", (0, 1, 2), None)
+    x, w = torch.zeros(1, 2, 8, dtype=BF), torch.zeros(8, dtype=BF)
+    for args in [(x, w), (x, w, 1.0, 2), (x, w, 1.0), (x, 3, 1.0), (None, w, 1.0), (x, w, "a"),
+                 (torch.nn.Buffer(x), w, 1.0)]:
+        assert native.call(plan, *args) is False
+
+
+@pytest.mark.gpu
+def test_plain_calls_skip_the_python_path(pkg, device, monkeypatch):
+    """With the ctypes launch disabled: plain calls of every kind of argument
+    (table, index with and without its batch dim, workspace, fixed size) still
+    launch, and calls that need a conversion or a check reach it."""
+    def no_launch(*args):
+        raise AssertionError("python path")
+
+    gen = torch.Generator("cpu").manual_seed(3)
+    r = lambda *s: torch.randn(*s, generator=gen).to(BF).to(device)
+    x, y, w, out = r(1, 9, 520), r(1, 9, 520), r(520), torch.empty(1, 9, 520, dtype=BF, device=device)
+    tab, index = r(3, 520), torch.tensor([0, 0, 1, 1, 1, 2, 2, 2, 2], device=device)
+    q, k, v = (r(7, 1, 2, 128) for _ in range(3))
+    outs = [torch.empty_like(q) for _ in range(3)]
+    cache, w128, pos = r(7, 96), r(128), torch.arange(7, device=device)
+    att = [r(1, 2, 300, 128) for _ in range(3)] + [0.1, torch.empty(1, 2, 300, 128, dtype=BF, device=device)]
+    attention = pkg.make_attention()
+    attention(*att)  # plans the shape
+    want_att = att[4].clone()
+    swiglu, rms = pkg.make_swiglu(), pkg.make_rms(width=520)
+    mod, pack = pkg.make_rms_modulate_indexed(check_indices=False), pkg.make_qkv_norm_rope_pack()
+    mod(x, w, EPS, tab, tab, index, out)
+    want_mod = out.clone()
+    pack(q, k, v, w128, w128, EPS, cache, pos.int(), *outs)  # int32 positions: converted in Python
+    want_pack = [t.clone() for t in outs]
+    monkeypatch.setattr(pkg._lib, "launch", no_launch)
+    swiglu(x, y, out)
+    rms(x, w, 0, out)
+    for ix in (index, index.view(1, 9)):
+        out.zero_()
+        mod(x, w, EPS, tab, tab, ix, out)
+        assert torch.equal(out, want_mod)
+    for t in outs:
+        t.zero_()
+    pack(q, k, v, w128, w128, EPS, cache, pos, *outs)
+    assert all(torch.equal(a, b) for a, b in zip(outs, want_pack))
+    att[4].zero_()
+    attention(*att)
+    assert torch.equal(att[4], want_att)
+    for call in [lambda: pack(q, k, v, w128, w128, EPS, cache, pos.int(), *outs),
+                 lambda: rms(x, w, torch.tensor(EPS), out),
+                 lambda: swiglu(torch.nn.Parameter(x).view(1, 9, 520).as_subclass(_Sub), y, out)]:
+        with pytest.raises(AssertionError, match="python path"):
+            call()
+    for call in [lambda: rms(r(1, 9, 128), r(128), EPS, r(1, 9, 128)), lambda: swiglu(x.float(), y, out),
+                 lambda: swiglu(x[0], y, out), lambda: swiglu(x.cpu(), y, out),
+                 lambda: attention(att[0][..., :64], *att[1:])]:
+        with pytest.raises(ValueError):
+            call()
+
+
+class _Sub(torch.Tensor):
+    pass
+
+
+@pytest.mark.gpu
+def test_calls_use_the_current_stream(pkg, device):
+    """A call under a side stream is captured there."""
+    x = torch.randn(1, 64, 1024, device=device).to(BF)
+    out = torch.zeros_like(x)
+    swiglu = pkg.make_swiglu()
+    swiglu(x, x, out)
+    torch.cuda.synchronize()
+    want = out.clone()
+    graph, side = torch.cuda.CUDAGraph(), torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        with torch.cuda.graph(graph, stream=side):
+            swiglu(x, x, out)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.equal(out, want)
