@@ -1369,28 +1369,25 @@ __device__ __forceinline__ void head_rms(float f[8], const float w[8], float eps
 
 // Rotate-half RoPE on channels 0..95 (pairs i, i+48), 96..127 pass through,
 // cos/sin [T, 48] (tools/h3_pointwise.py:199-214). Lanes 0-5 hold the first
-// halves, lanes 6-11 the second halves, lanes 12-15 the pass-through.
+// halves a, lanes 6-11 the second halves b, lanes 12-15 the pass-through. A
+// lane's output is bf16(own c) + bf16(partner s') in both halves -- (a c) + (-b s)
+// and (b c) + (a s) -- with s' = -s in the first: negating the packed table
+// entry once (four XORs) instead of choosing a, b and the products per element
+// takes 32 of a row's VALU instructions out: q and k at 8192 tokens of 14 heads,
+// one launch each, 29.3 -> 27.8 us; the q/k/v pack 37.1 -> 36.5 us.
 __device__ __forceinline__ void rope_rotate_half(float f[8], int lane, const RopeTab &tab) {
     float partner[8];
     const int src = lane < 6 ? lane + 6 : (lane < 12 ? lane - 6 : lane);
 #pragma unroll
     for (int e = 0; e < 8; ++e) partner[e] = __shfl(f[e], src, 16);
     if (lane >= 12) return;
+    const uint32_t flip = lane < 6 ? 0x80008000u : 0u;
     float c[8], s[8];
     u4_to_f8(tab.c, c);
-    u4_to_f8(tab.s, s);
+    u4_to_f8({tab.s.x ^ flip, tab.s.y ^ flip, tab.s.z ^ flip, tab.s.w ^ flip}, s);
 #pragma unroll
     for (int e = 0; e < 8; ++e) {
-        const float av = lane < 6 ? f[e] : partner[e];  // first half a
-        const float bv = lane < 6 ? partner[e] : f[e];  // second half b
-        float t0, t1;
-        if (lane < 6) {
-            t0 = av * c[e];     // ac = bf16(a c)
-            t1 = -bv * s[e];    // bs = bf16(-b s)
-        } else {
-            t0 = bv * c[e];     // bc = bf16(b c)
-            t1 = av * s[e];     // as = bf16(a s)
-        }
+        float t0 = f[e] * c[e], t1 = partner[e] * s[e];
         rbf2(t0, t1);
         f[e] = t0 + t1;  // y = bf16(. + .), rounded by the store
     }
@@ -1539,6 +1536,17 @@ __global__ __launch_bounds__(kThreads) void head_rows_loop_kernel(RopeArgs a) {
 // (interleaved) and 14.4-15.0 against 15.1-16.3 us (rotate-half) per tensor.
 constexpr int kHeadLoopBlocks = 4096;
 constexpr int kHeadLoopRows = 1;
+// Blocks of a persistent head-row launch: `least`, or more where they would
+// take more than `turns` batches each, up to `most`. q and k in one launch
+// (4096 to 8192 blocks, 4 turns) at 18,000 tokens of 28 heads: 94.8 us over 4096
+// blocks, 91.1 over 8192; 8192 tokens of 14 heads: 24.4 and 25.3. The pack (2048
+// to 4096 blocks, 5 turns) at 5726 tokens of 56 heads: 94.8 us over 2048, 92.6
+// over 4096; 8192 tokens of 14 heads: 37.0 and 39.9.
+int64_t head_blocks(int64_t batches, int64_t least, int64_t most, int64_t turns) {
+    int64_t n = batches / turns;
+    n = n < least ? least : (n > most ? most : n);
+    return batches < n ? batches : n;
+}
 
 // x2 / out2 / w2 (optional, all or none): a second tensor of x's shape taken
 // in the same launch (one pass over both when the rows are 16-byte aligned and
@@ -1608,7 +1616,7 @@ int launch_head_rows(hipStream_t stream, const View<4> &x, const View<4> &out, c
     if (kHeadLoopBlocks > 0 && vec && off32) {
         constexpr int64_t kBatch = kPerBlock * kHeadLoopRows;
         const int64_t needed = (a.rows + kBatch - 1) / kBatch;
-        const unsigned gl = static_cast<unsigned>(needed < kHeadLoopBlocks ? needed : kHeadLoopBlocks);
+        const unsigned gl = static_cast<unsigned>(head_blocks(needed, kHeadLoopBlocks, 2 * kHeadLoopBlocks, 4));
         if (pair)
             head_rows_loop_kernel<true, MODE, kHeadLoopRows, true, 2><<<gl, kThreads, 0, stream>>>(a);
         else
@@ -2096,11 +2104,10 @@ int launch_qkv_pack(hipStream_t stream, const View<4> *in, const View<4> *out, c
     }
     if (rows >= (int64_t{1} << 31) - kThreads * 4) return kInvalid;
     if (check_only) return 0;
-    // kQkvBlocks blocks per tensor at most, one batch of kThreads / 16 rows each
-    // per turn.
+    // Blocks per tensor, one batch of kThreads / 16 rows each per turn.
     constexpr int64_t kBatch = kThreads / 16 * kQkvRows;
     const int64_t batches = (rows + kBatch - 1) / kBatch;
-    const int64_t tiles = batches < kQkvBlocks ? batches : kQkvBlocks;
+    const int64_t tiles = head_blocks(batches, kQkvBlocks, 2 * kQkvBlocks, 5);
     const int64_t heads = a.P * a.Hs;
     a.v_pinned = vamax && heads > 0 && tiles >= heads;
     if (vamax && !a.v_pinned) {  // the slots start at 0 (an empty V has amax 0)
