@@ -16,7 +16,8 @@
 //     16-byte chunks are XOR-swizzled so every operand read is bank-conflict
 //     free (below); the next tile's loads run during the current tile's work;
 //   - one workgroup fills a CU, so a launch runs in rounds of one workgroup
-//     per CU. When the last round would be about 2/3 to 3/4 full, it runs
+//     per CU. A launch of at most one round may run as smaller units
+//     (attention16_short_kernel). When the last round would be about 2/3 to 3/4 full, it runs
 //     instead as a full round of 192-query units (attention16_small_kernel).
 //     When it is otherwise partly filled and a workspace is given, the units
 //     of that round are split along the keys into pieces that fill whole
