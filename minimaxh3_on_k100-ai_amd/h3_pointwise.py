@@ -423,7 +423,8 @@ def make_qkv_norm_rope_pack_fp8x2_vamax(dtype=None):
 
     def kernel(q, k, v, q_weight, k_weight, eps, cache, positions, q8, q8_lo, k8, k8_lo, v_out, q_descale,
                k_descale, v_amax):
-        if fast(q, k, v, q_weight, k_weight, eps, cache, positions, q8, q8_lo, k8, k8_lo, v_out, q_descale,
+        if q8_lo.stride() == q8.stride() and k8_lo.stride() == k8.stride() and fast(
+                q, k, v, q_weight, k_weight, eps, cache, positions, q8, q8_lo, k8, k8_lo, v_out, q_descale,
                 k_descale, v_amax):
             return
         _ndim(4, q8_lo=q8_lo, k8_lo=k8_lo)

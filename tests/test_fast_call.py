@@ -86,6 +86,21 @@ def test_plain_calls_skip_the_python_path(pkg, device, monkeypatch):
             call()
 
 
+@pytest.mark.gpu
+def test_lo_code_strides_are_still_compared(pkg, device):
+    """The two-term pack refuses lo codes whose strides differ from the hi
+    codes', also where they only differ in a dim of size 1."""
+    r = lambda *s: torch.randn(*s, device=device).to(BF)
+    q, k, v = (r(5, 1, 2, 128) for _ in range(3))
+    codes = [torch.empty(5, 1, 2, 128, dtype=torch.float8_e4m3fn, device=device) for _ in range(4)]
+    codes[1] = codes[1].as_strided((5, 1, 2, 128), (256, 512, 128, 1))
+    d, amax = torch.empty(2, device=device), torch.empty(2, 64, device=device)
+    with pytest.raises(ValueError, match="strides"):
+        pkg.make_qkv_norm_rope_pack_fp8x2_vamax()(q, k, v, r(128), r(128), EPS, r(5, 96),
+                                                  torch.arange(5, device=device), *codes, torch.empty_like(v), d,
+                                                  d.clone(), amax)
+
+
 class _Sub(torch.Tensor):
     pass
 
