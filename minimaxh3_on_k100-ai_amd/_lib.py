@@ -122,11 +122,14 @@ def _not_taken(*args) -> bool:
 
 
 def fast(name: str, kinds: str, order: tuple | None = None, fix: tuple | None = None):
-    """A callable that launches entry point `name` when every argument is as
+    """A callable that calls entry point `name` once when every argument is as
     `kinds` says (csrc/h3_call.cpp: a kind and a rank per argument) and returns
-    whether it did. order: the launcher's arguments by index of the call's;
-    fix: (argument, dim, size) that must hold. Without the library it takes no
-    call, and the ctypes path raises at first use."""
+    True, or its status where that is not 0; False if it did not call it. Unless
+    True, the ctypes path runs the checks and hands the result on to
+    `launch_after`, which raises a status and launches after False. order: the launcher's
+    arguments by index of the call's; fix: (argument, dim, size) that must hold.
+    Without the library it takes no call, and the ctypes path raises at first
+    use."""
     key = (name, kinds, order, fix)
     bound = _fast_calls.get(key)
     if bound is None:
@@ -228,6 +231,14 @@ def launch(name: str, device: torch.device, *args: _Arg) -> None:
         status = call(name, stream, *args)
     if status != 0:
         raise LaunchError(name, status)
+
+
+def launch_after(status: bool | int, name: str, device: torch.device, *args: _Arg) -> None:
+    """`launch` of what `fast` did not call (status False); raises the status of
+    what it did, without launching again."""
+    if status is not False:
+        raise LaunchError(name, status)
+    launch(name, device, *args)
 
 
 def check_cuda(*tensors: torch.Tensor) -> torch.device:

@@ -7,11 +7,13 @@
 // q/k/v pack, twelve) per call, most of it longer than the kernels of a
 // 256-token block. Here a call takes the launch itself and under 2 us.
 //
-// call(plan, *args) returns True when it launched. Anything but the plain case
-// -- every tensor an exact torch.Tensor on the current GPU with the planned
-// rank and dtype, the launcher's own checks passed -- returns False with
-// nothing launched, and the caller takes its Python path, which converts what
-// can be converted and raises what has to be raised.
+// call(plan, *args) calls the launcher once and returns True, or its status
+// where that is not 0. It returns False without having called it for anything
+// but the plain case (every tensor an exact torch.Tensor on the current GPU
+// with the planned rank and dtype): the caller takes its Python path, which
+// converts what can be converted and launches. After a status the caller must
+// not launch again: a launcher ends with the thread's last HIP error, which an
+// earlier call may have left, so its kernels may be queued all the same.
 #define PY_SSIZE_T_CLEAN
 #include <Python.h>
 
@@ -231,13 +233,13 @@ PyObject *call(PyObject *, PyObject *const *argv, Py_ssize_t nargs) {
     status = invoke(plan->fn, stream, a, m, std::make_index_sequence<kMaxArgs + 1>{});
     Py_END_ALLOW_THREADS
     if (status == 0) Py_RETURN_TRUE;
-    Py_RETURN_FALSE;
+    return PyLong_FromLong(status);
 }
 
 PyMethodDef methods[] = {
     {"plan", make_plan, METH_VARARGS, "plan(address, kinds, order, fix) -> launch plan"},
     {"call", reinterpret_cast<PyCFunction>(reinterpret_cast<void (*)()>(call)), METH_FASTCALL,
-     "call(plan, *args) -> whether it launched"},
+     "call(plan, *args) -> True, or the launcher's non-zero status; False if it was not called"},
     {nullptr, nullptr, 0, nullptr}};
 
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_h3call", "fast calls into libh3mi355x.so", -1, methods,

@@ -96,10 +96,11 @@ def make_attention(block_m=128, block_n=32, num_warps=4, num_stages=1, caller="t
 
     if not split:
         def kernel(q, k, v, scale, out):
-            if fast(q, k, v, scale, out):
+            status = fast(q, k, v, scale, out)
+            if status is True:
                 return
-            _lib.launch(entry, check(q, k, v, out), _lib.tensor(q), _lib.tensor(k), _lib.tensor(v),
-                        _lib.scalar(scale), _lib.tensor(out))
+            _lib.launch_after(status, entry, check(q, k, v, out), _lib.tensor(q), _lib.tensor(k), _lib.tensor(v),
+                              _lib.scalar(scale), _lib.tensor(out))
 
         return kernel
 
@@ -112,13 +113,14 @@ def make_attention(block_m=128, block_n=32, num_warps=4, num_stages=1, caller="t
             device = check(q, k, v, out)
             nbytes = workspaces[key] = _lib.planned_workspace(device.index, *q.shape[:3], k.shape[2], head_dim)
         ws = None if nbytes == 0 else torch.empty(nbytes, dtype=torch.uint8, device=q.device)
-        if fast(q, k, v, scale, out, ws):
+        status = fast(q, k, v, scale, out, ws)
+        if status is True:
             return
         device = check(q, k, v, out)
         if ws is None:
             ws = torch.empty(0, dtype=torch.uint8, device=device)
-        _lib.launch("launch_h3_attention_planned", device, _lib.tensor(q), _lib.tensor(k), _lib.tensor(v),
-                    _lib.scalar(scale), _lib.tensor(out), _lib.tensor(ws))
+        _lib.launch_after(status, "launch_h3_attention_planned", device, _lib.tensor(q), _lib.tensor(k),
+                          _lib.tensor(v), _lib.scalar(scale), _lib.tensor(out), _lib.tensor(ws))
 
     return kernel
 
@@ -138,8 +140,11 @@ def quantize_fp8_per_head(x: torch.Tensor, transposed: bool = False, x8: torch.T
     amax_slots: fp32 [H, 64] per-head maxima of |x| already folded by the
     producer (make_qkv_norm_rope_pack_fp8_vamax); then only the code pass
     reads x."""
-    if amax_slots is not None and x8 is not None and descale is not None and _slots_fast()(x, amax_slots, x8, descale):
-        return x8, descale
+    status = False
+    if amax_slots is not None and x8 is not None and descale is not None:
+        status = _slots_fast()(x, amax_slots, x8, descale)
+        if status is True:
+            return x8, descale
     if x.dim() != 4:
         raise ValueError("x must be [B, H, S, D]")
     device = _lib.check_cuda(x)
@@ -163,8 +168,8 @@ def quantize_fp8_per_head(x: torch.Tensor, transposed: bool = False, x8: torch.T
         _lib.check_dtype(torch.float32, amax_slots)
         if amax_slots.shape != (H, _lib.AMAX_SLOTS) or not amax_slots.is_contiguous():
             raise ValueError(f"amax_slots must be a contiguous fp32 [H, {_lib.AMAX_SLOTS}] tensor")
-        _lib.launch("launch_h3_quantize_fp8_per_head_slots", device, _lib.tensor(x), _lib.tensor(amax_slots),
-                    _lib.tensor(x8.view(torch.uint8)), _lib.tensor(descale))
+        _lib.launch_after(status, "launch_h3_quantize_fp8_per_head_slots", device, _lib.tensor(x),
+                          _lib.tensor(amax_slots), _lib.tensor(x8.view(torch.uint8)), _lib.tensor(descale))
         return x8, descale
     _lib.launch("launch_h3_quantize_fp8_per_head", device, _lib.tensor(x), _lib.tensor(x8.view(torch.uint8)),
                 _lib.tensor(descale))
@@ -186,17 +191,17 @@ def make_attention_fp8():
     fast = _lib.fast("launch_h3_full_attention_fp8", "e4e4e4c1c1c1s0b4")
 
     def kernel(q8, k8, v8, q_descale, k_descale, v_descale, scale, out):
-        if fast(q8, k8, v8, q_descale, k_descale, v_descale, scale, out):
+        status = fast(q8, k8, v8, q_descale, k_descale, v_descale, scale, out)
+        if status is True:
             return
         _check_qkvo(q8, k8, v8, out)
         device = _lib.check_cuda(q8, k8, v8, q_descale, k_descale, v_descale, out)
         _lib.check_dtype(torch.float8_e4m3fn, q8, k8, v8)
         _lib.check_dtype(torch.bfloat16, out)
         _check_descales(q8.shape[1], q_descale, k_descale, v_descale)
-        _lib.launch("launch_h3_full_attention_fp8", device, _lib.tensor(q8.view(torch.uint8)),
-                    _lib.tensor(k8.view(torch.uint8)), _lib.tensor(v8.view(torch.uint8)),
-                    _lib.tensor(q_descale), _lib.tensor(k_descale), _lib.tensor(v_descale),
-                    _lib.scalar(scale), _lib.tensor(out))
+        _lib.launch_after(status, "launch_h3_full_attention_fp8", device, _lib.tensor(q8.view(torch.uint8)),
+                          _lib.tensor(k8.view(torch.uint8)), _lib.tensor(v8.view(torch.uint8)), _lib.tensor(q_descale),
+                          _lib.tensor(k_descale), _lib.tensor(v_descale), _lib.scalar(scale), _lib.tensor(out))
 
     return kernel
 
@@ -237,7 +242,8 @@ def make_attention_fp8x2():
     fast = _lib.fast("launch_h3_full_attention_fp8x2", "e4e4e4e4e4c1c1c1s0b4")
 
     def kernel(q8, q8_lo, k8, k8_lo, v8, q_descale, k_descale, v_descale, scale, out):
-        if fast(q8, q8_lo, k8, k8_lo, v8, q_descale, k_descale, v_descale, scale, out):
+        status = fast(q8, q8_lo, k8, k8_lo, v8, q_descale, k_descale, v_descale, scale, out)
+        if status is True:
             return
         _check_qkvo(q8, k8, v8, out)
         if q8_lo.shape != q8.shape or k8_lo.shape != k8.shape:
@@ -246,10 +252,10 @@ def make_attention_fp8x2():
         _lib.check_dtype(torch.float8_e4m3fn, q8, q8_lo, k8, k8_lo, v8)
         _lib.check_dtype(torch.bfloat16, out)
         _check_descales(q8.shape[1], q_descale, k_descale, v_descale)
-        _lib.launch("launch_h3_full_attention_fp8x2", device, *(_lib.tensor(t.view(torch.uint8))
-                                                                for t in (q8, q8_lo, k8, k8_lo, v8)),
-                    _lib.tensor(q_descale), _lib.tensor(k_descale), _lib.tensor(v_descale), _lib.scalar(scale),
-                    _lib.tensor(out))
+        _lib.launch_after(status, "launch_h3_full_attention_fp8x2", device,
+                          *(_lib.tensor(t.view(torch.uint8)) for t in (q8, q8_lo, k8, k8_lo, v8)),
+                          _lib.tensor(q_descale), _lib.tensor(k_descale), _lib.tensor(v_descale), _lib.scalar(scale),
+                          _lib.tensor(out))
 
     return kernel
 
@@ -261,15 +267,16 @@ def make_attention_fp8pv():
     fast = _lib.fast("launch_h3_full_attention_fp8pv", "b4b4e4c1s0b4")
 
     def kernel(q, k, v8, v_descale, scale, out):
-        if fast(q, k, v8, v_descale, scale, out):
+        status = fast(q, k, v8, v_descale, scale, out)
+        if status is True:
             return
         _check_qkvo(q, k, v8, out)
         device = _lib.check_cuda(q, k, v8, v_descale, out)
         _lib.check_dtype(torch.bfloat16, q, k, out)
         _lib.check_dtype(torch.float8_e4m3fn, v8)
         _check_descales(q.shape[1], v_descale)
-        _lib.launch("launch_h3_full_attention_fp8pv", device, _lib.tensor(q), _lib.tensor(k),
-                    _lib.tensor(v8.view(torch.uint8)), _lib.tensor(v_descale), _lib.scalar(scale),
-                    _lib.tensor(out))
+        _lib.launch_after(status, "launch_h3_full_attention_fp8pv", device, _lib.tensor(q), _lib.tensor(k),
+                          _lib.tensor(v8.view(torch.uint8)), _lib.tensor(v_descale), _lib.scalar(scale),
+                          _lib.tensor(out))
 
     return kernel

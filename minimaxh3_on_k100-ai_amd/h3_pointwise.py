@@ -52,11 +52,13 @@ def make_swiglu(caller="torch", output_dir=None, archs=None, rows=1, cols=1024, 
     fast = _lib.fast("launch_h3_swiglu_exact", "b3b3b3")
 
     def kernel(up, gate, out):
-        if fast(up, gate, out):
+        status = fast(up, gate, out)
+        if status is True:
             return
         _ndim(3, up=up, gate=gate, out=out)
         device = _bf16(up, gate, out)
-        _lib.launch("launch_h3_swiglu_exact", device, _lib.tensor(up), _lib.tensor(gate), _lib.tensor(out))
+        _lib.launch_after(status, "launch_h3_swiglu_exact", device, _lib.tensor(up), _lib.tensor(gate),
+                          _lib.tensor(out))
 
     return kernel
 
@@ -70,14 +72,16 @@ def make_rms(caller="torch", output_dir=None, archs=None, width=5376, dtype=None
     fast = _lib.fast(name, "b3b1s0b3", fix=None if width is None else (0, 2, width))
 
     def kernel(x, weight, eps, out):
-        if fast(x, weight, eps, out):
+        status = fast(x, weight, eps, out)
+        if status is True:
             return
         _ndim(3, x=x, out=out)
         _ndim(1, weight=weight)
         if width is not None and x.shape[-1] != width:
             raise ValueError(f"this kernel was made for width {width}, got {x.shape[-1]}")
         device = _bf16(x, weight, out)
-        _lib.launch(name, device, _lib.tensor(x), _lib.tensor(weight), _lib.scalar(eps), _lib.tensor(out))
+        _lib.launch_after(status, name, device, _lib.tensor(x), _lib.tensor(weight), _lib.scalar(eps),
+                          _lib.tensor(out))
 
     return kernel
 
@@ -89,13 +93,14 @@ def make_rms_modulate(caller="torch", output_dir=None, archs=None, dtype=None):
     fast = _lib.fast("launch_h3_rms_modulate_exact", "b3b1s0b3b3b3")
 
     def kernel(x, weight, eps, scale, shift, out):
-        if fast(x, weight, eps, scale, shift, out):
+        status = fast(x, weight, eps, scale, shift, out)
+        if status is True:
             return
         _ndim(3, x=x, scale=scale, shift=shift, out=out)
         _ndim(1, weight=weight)
         device = _bf16(x, weight, scale, shift, out)
-        _lib.launch("launch_h3_rms_modulate_exact", device, _lib.tensor(x), _lib.tensor(weight),
-                    _lib.scalar(eps), _lib.tensor(scale), _lib.tensor(shift), _lib.tensor(out))
+        _lib.launch_after(status, "launch_h3_rms_modulate_exact", device, _lib.tensor(x), _lib.tensor(weight),
+                          _lib.scalar(eps), _lib.tensor(scale), _lib.tensor(shift), _lib.tensor(out))
 
     return kernel
 
@@ -106,12 +111,13 @@ def make_gated_residual(caller="torch", output_dir=None, archs=None, block=(4, 5
     fast = _lib.fast("launch_h3_gated_residual_exact", "b3b3b3b3")
 
     def kernel(x, gate, y, out):
-        if fast(x, gate, y, out):
+        status = fast(x, gate, y, out)
+        if status is True:
             return
         _ndim(3, x=x, gate=gate, y=y, out=out)
         device = _bf16(x, gate, y, out)
-        _lib.launch("launch_h3_gated_residual_exact", device, _lib.tensor(x), _lib.tensor(gate),
-                    _lib.tensor(y), _lib.tensor(out))
+        _lib.launch_after(status, "launch_h3_gated_residual_exact", device, _lib.tensor(x), _lib.tensor(gate),
+                          _lib.tensor(y), _lib.tensor(out))
 
     return kernel
 
@@ -123,14 +129,15 @@ def make_gated_residual_rms_modulate(caller="torch", output_dir=None, archs=None
     fast = _lib.fast("launch_h3_gated_residual_rms_modulate_exact", "b3b3b3b1s0b3b3b3b3")
 
     def kernel(x, gate, y, weight, eps, scale, shift, residual, out):
-        if fast(x, gate, y, weight, eps, scale, shift, residual, out):
+        status = fast(x, gate, y, weight, eps, scale, shift, residual, out)
+        if status is True:
             return
         _ndim(3, x=x, gate=gate, y=y, scale=scale, shift=shift, residual=residual, out=out)
         _ndim(1, weight=weight)
         device = _bf16(x, gate, y, weight, scale, shift, residual, out)
-        _lib.launch("launch_h3_gated_residual_rms_modulate_exact", device, _lib.tensor(x), _lib.tensor(gate),
-                    _lib.tensor(y), _lib.tensor(weight), _lib.scalar(eps), _lib.tensor(scale),
-                    _lib.tensor(shift), _lib.tensor(residual), _lib.tensor(out))
+        _lib.launch_after(status, "launch_h3_gated_residual_rms_modulate_exact", device, _lib.tensor(x),
+                          _lib.tensor(gate), _lib.tensor(y), _lib.tensor(weight), _lib.scalar(eps), _lib.tensor(scale),
+                          _lib.tensor(shift), _lib.tensor(residual), _lib.tensor(out))
 
     return kernel
 
@@ -188,16 +195,17 @@ def make_rms_modulate_indexed(check_indices: bool = True):
     fast = _lib.fast("launch_h3_rms_modulate_indexed", "b3b1s0b2b2i2b3")
 
     def kernel(x, weight, eps, scale, shift, index, out):
-        if not check_indices and fast(x, weight, eps, scale, shift, index, out):
+        status = False if check_indices else fast(x, weight, eps, scale, shift, index, out)
+        if status is True:
             return
         _ndim(3, x=x, out=out)
         _ndim(2, scale=scale, shift=shift)
         _ndim(1, weight=weight)
         device = _bf16(x, weight, scale, shift, out)
         index = _token_index(index, x, scale.shape[0], check_indices)
-        _lib.launch("launch_h3_rms_modulate_indexed", device, _lib.tensor(x), _lib.tensor(weight),
-                    _lib.scalar(eps), _lib.tensor(scale), _lib.tensor(shift), _lib.tensor(index),
-                    _lib.tensor(out))
+        _lib.launch_after(status, "launch_h3_rms_modulate_indexed", device, _lib.tensor(x), _lib.tensor(weight),
+                          _lib.scalar(eps), _lib.tensor(scale), _lib.tensor(shift), _lib.tensor(index),
+                          _lib.tensor(out))
 
     return kernel
 
@@ -209,16 +217,17 @@ def make_gated_residual_rms_modulate_indexed(check_indices: bool = True):
     fast = _lib.fast("launch_h3_gated_residual_rms_modulate_indexed", "b3b2b3b1s0b2b2i2b3b3")
 
     def kernel(x, gate, y, weight, eps, scale, shift, index, residual, out):
-        if not check_indices and fast(x, gate, y, weight, eps, scale, shift, index, residual, out):
+        status = False if check_indices else fast(x, gate, y, weight, eps, scale, shift, index, residual, out)
+        if status is True:
             return
         _ndim(3, x=x, y=y, residual=residual, out=out)
         _ndim(2, gate=gate, scale=scale, shift=shift)
         _ndim(1, weight=weight)
         device = _bf16(x, gate, y, weight, scale, shift, residual, out)
         index = _token_index(index, x, scale.shape[0], check_indices)
-        _lib.launch("launch_h3_gated_residual_rms_modulate_indexed", device, _lib.tensor(x), _lib.tensor(gate),
-                    _lib.tensor(y), _lib.tensor(weight), _lib.scalar(eps), _lib.tensor(scale),
-                    _lib.tensor(shift), _lib.tensor(index), _lib.tensor(residual), _lib.tensor(out))
+        _lib.launch_after(status, "launch_h3_gated_residual_rms_modulate_indexed", device, _lib.tensor(x),
+                          _lib.tensor(gate), _lib.tensor(y), _lib.tensor(weight), _lib.scalar(eps), _lib.tensor(scale),
+                          _lib.tensor(shift), _lib.tensor(index), _lib.tensor(residual), _lib.tensor(out))
 
     return kernel
 
@@ -229,14 +238,15 @@ def make_gated_residual_indexed(check_indices: bool = True):
     fast = _lib.fast("launch_h3_gated_residual_indexed", "b3b2b3i2b3")
 
     def kernel(x, gate, y, index, out):
-        if not check_indices and fast(x, gate, y, index, out):
+        status = False if check_indices else fast(x, gate, y, index, out)
+        if status is True:
             return
         _ndim(3, x=x, y=y, out=out)
         _ndim(2, gate=gate)
         device = _bf16(x, gate, y, out)
         index = _token_index(index, x, gate.shape[0], check_indices)
-        _lib.launch("launch_h3_gated_residual_indexed", device, _lib.tensor(x), _lib.tensor(gate),
-                    _lib.tensor(y), _lib.tensor(index), _lib.tensor(out))
+        _lib.launch_after(status, "launch_h3_gated_residual_indexed", device, _lib.tensor(x), _lib.tensor(gate),
+                          _lib.tensor(y), _lib.tensor(index), _lib.tensor(out))
 
     return kernel
 
@@ -248,25 +258,31 @@ def make_rope(caller="torch", output_dir=None, archs=None, dtype=None):
     fast = _lib.fast("launch_h3_rope_exact", "b3b2b2b3", (0, 0, 0, 1, 2, 3, 3, 3))
 
     def launch(x, cos, sin, out):
-        if fast(x, cos, sin, out):
+        status = fast(x, cos, sin, out)
+        if status is True:
             return
         _ndim(3, x=x, out=out)
         _ndim(2, cos=cos, sin=sin)
         device = _bf16(x, cos, sin, out)
         xa, oa = _lib.tensor(x), _lib.tensor(out)
-        _lib.launch("launch_h3_rope_exact", device, xa, xa, xa, _lib.tensor(cos), _lib.tensor(sin), oa, oa, oa)
+        _lib.launch_after(status, "launch_h3_rope_exact", device, xa, xa, xa, _lib.tensor(cos), _lib.tensor(sin), oa,
+                          oa, oa)
 
     return launch
 
 
-def _qk_raw(x0, x1, xp, w0, w1, wp, eps, cos, sin, y0, y1, yp):
+def _qk_launch(x0, x1, xp, w0, w1, wp, eps, cos, sin, y0, y1, yp, status=False):
     _ndim(4, x0=x0, x1=x1, xp=xp, y0=y0, y1=y1, yp=yp)
     _ndim(1, w0=w0, w1=w1, wp=wp)
     _ndim(2, cos=cos, sin=sin)
     device = _bf16(x0, x1, xp, w0, w1, wp, cos, sin, y0, y1, yp)
-    _lib.launch("launch_h3_qk_norm_rope", device, _lib.tensor(x0), _lib.tensor(x1), _lib.tensor(xp),
-                _lib.tensor(w0), _lib.tensor(w1), _lib.tensor(wp), _lib.scalar(eps), _lib.tensor(cos),
-                _lib.tensor(sin), _lib.tensor(y0), _lib.tensor(y1), _lib.tensor(yp))
+    _lib.launch_after(status, "launch_h3_qk_norm_rope", device, _lib.tensor(x0), _lib.tensor(x1), _lib.tensor(xp),
+                      _lib.tensor(w0), _lib.tensor(w1), _lib.tensor(wp), _lib.scalar(eps), _lib.tensor(cos),
+                      _lib.tensor(sin), _lib.tensor(y0), _lib.tensor(y1), _lib.tensor(yp))
+
+
+def _qk_raw(x0, x1, xp, w0, w1, wp, eps, cos, sin, y0, y1, yp):
+    _qk_launch(x0, x1, xp, w0, w1, wp, eps, cos, sin, y0, y1, yp)
 
 
 def make_qk_norm_rope(caller="torch", output_dir=None, archs=None, rows=8, num_warps=1, block_tokens=1, ranks=1,
@@ -284,9 +300,10 @@ def make_qk_norm_rope(caller="torch", output_dir=None, archs=None, rows=8, num_w
     fast = _lib.fast("launch_h3_qk_norm_rope", "b4b1s0b2b2b4", (0, 0, 0, 1, 1, 1, 2, 3, 4, 5, 5, 5))
 
     def launch(x, weight, eps, cos, sin, out):
-        if fast(x, weight, eps, cos, sin, out):
+        status = fast(x, weight, eps, cos, sin, out)
+        if status is True:
             return
-        _qk_raw(x, x, x, weight, weight, weight, eps, cos, sin, out, out, out)
+        _qk_launch(x, x, x, weight, weight, weight, eps, cos, sin, out, out, out, status)
 
     return launch
 
@@ -319,7 +336,8 @@ def make_qkv_norm_rope_pack(dtype=None):
     fast = _lib.fast("launch_h3_qkv_norm_rope_pack", "b4b4b4b1b1s0t2l1b4b4b4")
 
     def kernel(q, k, v, q_weight, k_weight, eps, cache, positions, q_out, k_out, v_out):
-        if fast(q, k, v, q_weight, k_weight, eps, cache, positions, q_out, k_out, v_out):
+        status = fast(q, k, v, q_weight, k_weight, eps, cache, positions, q_out, k_out, v_out)
+        if status is True:
             return
         _ndim(4, q=q, k=k, v=v, q_out=q_out, k_out=k_out, v_out=v_out)
         _ndim(1, q_weight=q_weight, k_weight=k_weight, positions=positions)
@@ -331,10 +349,10 @@ def make_qkv_norm_rope_pack(dtype=None):
             raise ValueError("positions must be an int32 or int64 tensor on the device of q")
         if positions.dtype != torch.int64:
             positions = positions.to(torch.int64)
-        _lib.launch("launch_h3_qkv_norm_rope_pack", device, _lib.tensor(q), _lib.tensor(k), _lib.tensor(v),
-                    _lib.tensor(q_weight), _lib.tensor(k_weight), _lib.scalar(eps), _lib.tensor(cache[:, :48]),
-                    _lib.tensor(cache[:, 48:]), _lib.tensor(positions), _lib.tensor(q_out), _lib.tensor(k_out),
-                    _lib.tensor(v_out))
+        _lib.launch_after(status, "launch_h3_qkv_norm_rope_pack", device, _lib.tensor(q), _lib.tensor(k),
+                          _lib.tensor(v), _lib.tensor(q_weight), _lib.tensor(k_weight), _lib.scalar(eps),
+                          _lib.tensor(cache[:, :48]), _lib.tensor(cache[:, 48:]), _lib.tensor(positions),
+                          _lib.tensor(q_out), _lib.tensor(k_out), _lib.tensor(v_out))
 
     return kernel
 
@@ -358,10 +376,11 @@ def make_qkv_norm_rope_pack_fp8(dtype=None):
     fast = _lib.fast("launch_h3_qkv_norm_rope_pack_fp8", "b4b4b4b1b1s0t2l1u4u4b4f1f1")
 
     def kernel(q, k, v, q_weight, k_weight, eps, cache, positions, q8, k8, v_out, q_descale, k_descale,
-               _entry="launch_h3_qkv_norm_rope_pack_fp8", _extra=()):
-        if not _extra and fast(q, k, v, q_weight, k_weight, eps, cache, positions, q8, k8, v_out, q_descale,
-                               k_descale):
-            return
+               _entry="launch_h3_qkv_norm_rope_pack_fp8", _extra=(), _status=False):
+        if not _extra:
+            _status = fast(q, k, v, q_weight, k_weight, eps, cache, positions, q8, k8, v_out, q_descale, k_descale)
+            if _status is True:
+                return
         _ndim(4, q=q, k=k, v=v, q8=q8, k8=k8, v_out=v_out)
         _ndim(1, q_weight=q_weight, k_weight=k_weight, positions=positions, q_descale=q_descale,
               k_descale=k_descale)
@@ -375,10 +394,10 @@ def make_qkv_norm_rope_pack_fp8(dtype=None):
                 raise ValueError(f"{name} must be float8_e4m3fn or uint8, got {t.dtype}")
         _lib.check_dtype(torch.float32, q_descale, k_descale)
         positions = _positions(positions, device)
-        _lib.launch(_entry, device, _lib.tensor(q), _lib.tensor(k), _lib.tensor(v),
-                    _lib.tensor(q_weight), _lib.tensor(k_weight), _lib.scalar(eps), _lib.tensor(cache[:, :48]),
-                    _lib.tensor(cache[:, 48:]), _lib.tensor(positions), _lib.tensor(q8), _lib.tensor(k8),
-                    _lib.tensor(v_out), _lib.tensor(q_descale), _lib.tensor(k_descale), *_extra)
+        _lib.launch_after(_status, _entry, device, _lib.tensor(q), _lib.tensor(k), _lib.tensor(v),
+                          _lib.tensor(q_weight), _lib.tensor(k_weight), _lib.scalar(eps), _lib.tensor(cache[:, :48]),
+                          _lib.tensor(cache[:, 48:]), _lib.tensor(positions), _lib.tensor(q8), _lib.tensor(k8),
+                          _lib.tensor(v_out), _lib.tensor(q_descale), _lib.tensor(k_descale), *_extra)
 
     return kernel
 
@@ -397,7 +416,8 @@ def make_qkv_norm_rope_pack_fp8_vamax(dtype=None):
     fast = _lib.fast("launch_h3_qkv_norm_rope_pack_fp8_vamax", "b4b4b4b1b1s0t2l1u4u4b4f1f1c2")
 
     def kernel(q, k, v, q_weight, k_weight, eps, cache, positions, q8, k8, v_out, q_descale, k_descale, v_amax):
-        if fast(q, k, v, q_weight, k_weight, eps, cache, positions, q8, k8, v_out, q_descale, k_descale, v_amax):
+        status = fast(q, k, v, q_weight, k_weight, eps, cache, positions, q8, k8, v_out, q_descale, k_descale, v_amax)
+        if status is True:
             return
         _ndim(2, v_amax=v_amax)
         _lib.check_cuda(q, v_amax)
@@ -406,7 +426,8 @@ def make_qkv_norm_rope_pack_fp8_vamax(dtype=None):
         if v_amax.shape != (heads, _lib.AMAX_SLOTS) or not v_amax.is_contiguous():
             raise ValueError(f"v_amax must be a contiguous fp32 [{heads}, {_lib.AMAX_SLOTS}] tensor")
         base(q, k, v, q_weight, k_weight, eps, cache, positions, q8, k8, v_out, q_descale, k_descale,
-             _entry="launch_h3_qkv_norm_rope_pack_fp8_vamax", _extra=(_lib.tensor(v_amax),))
+             _entry="launch_h3_qkv_norm_rope_pack_fp8_vamax", _extra=(_lib.tensor(v_amax),),
+             _status=status)
 
     return kernel
 
@@ -423,10 +444,12 @@ def make_qkv_norm_rope_pack_fp8x2_vamax(dtype=None):
 
     def kernel(q, k, v, q_weight, k_weight, eps, cache, positions, q8, q8_lo, k8, k8_lo, v_out, q_descale,
                k_descale, v_amax):
-        if q8_lo.stride() == q8.stride() and k8_lo.stride() == k8.stride() and fast(
-                q, k, v, q_weight, k_weight, eps, cache, positions, q8, q8_lo, k8, k8_lo, v_out, q_descale,
-                k_descale, v_amax):
-            return
+        status = False
+        if q8_lo.stride() == q8.stride() and k8_lo.stride() == k8.stride():
+            status = fast(q, k, v, q_weight, k_weight, eps, cache, positions, q8, q8_lo, k8, k8_lo, v_out, q_descale,
+                          k_descale, v_amax)
+            if status is True:
+                return
         _ndim(4, q8_lo=q8_lo, k8_lo=k8_lo)
         _ndim(2, v_amax=v_amax)
         _lib.check_cuda(q, q8_lo, k8_lo, v_amax)
@@ -452,11 +475,11 @@ def make_qkv_norm_rope_pack_fp8x2_vamax(dtype=None):
                 raise ValueError(f"{name} must be float8_e4m3fn or uint8, got {t.dtype}")
         _lib.check_dtype(torch.float32, q_descale, k_descale)
         positions = _positions(positions, device)
-        _lib.launch("launch_h3_qkv_norm_rope_pack_fp8x2_vamax", device, _lib.tensor(q), _lib.tensor(k),
-                    _lib.tensor(v), _lib.tensor(q_weight), _lib.tensor(k_weight), _lib.scalar(eps),
-                    _lib.tensor(cache[:, :48]), _lib.tensor(cache[:, 48:]), _lib.tensor(positions), _lib.tensor(q8),
-                    _lib.tensor(q8_lo), _lib.tensor(k8), _lib.tensor(k8_lo), _lib.tensor(v_out),
-                    _lib.tensor(q_descale), _lib.tensor(k_descale), _lib.tensor(v_amax))
+        _lib.launch_after(status, "launch_h3_qkv_norm_rope_pack_fp8x2_vamax", device, _lib.tensor(q), _lib.tensor(k),
+                          _lib.tensor(v), _lib.tensor(q_weight), _lib.tensor(k_weight), _lib.scalar(eps),
+                          _lib.tensor(cache[:, :48]), _lib.tensor(cache[:, 48:]), _lib.tensor(positions),
+                          _lib.tensor(q8), _lib.tensor(q8_lo), _lib.tensor(k8), _lib.tensor(k8_lo), _lib.tensor(v_out),
+                          _lib.tensor(q_descale), _lib.tensor(k_descale), _lib.tensor(v_amax))
 
     return kernel
 
@@ -510,14 +533,15 @@ def make_qk_norm_rope_interleaved(dtype=None):
     fast = _lib.fast("launch_h3_qk_norm_rope_interleaved", "b4b1s0b2b2b4")
 
     def launch(x, weight, eps, cos, sin, out):
-        if fast(x, weight, eps, cos, sin, out):
+        status = fast(x, weight, eps, cos, sin, out)
+        if status is True:
             return
         _ndim(4, x=x, out=out)
         _ndim(1, weight=weight)
         _ndim(2, cos=cos, sin=sin)
         device = _bf16(x, weight, cos, sin, out)
-        _lib.launch("launch_h3_qk_norm_rope_interleaved", device, _lib.tensor(x), _lib.tensor(weight),
-                    _lib.scalar(eps), _lib.tensor(cos), _lib.tensor(sin), _lib.tensor(out))
+        _lib.launch_after(status, "launch_h3_qk_norm_rope_interleaved", device, _lib.tensor(x), _lib.tensor(weight),
+                          _lib.scalar(eps), _lib.tensor(cos), _lib.tensor(sin), _lib.tensor(out))
 
     return launch
 
@@ -531,15 +555,16 @@ def make_qk_norm_rope_interleaved_qk(dtype=None):
     fast = _lib.fast("launch_h3_qk_norm_rope_interleaved_qk", "b4b4b1b1s0b2b2b4b4")
 
     def launch(q, k, q_weight, k_weight, eps, cos, sin, q_out, k_out):
-        if fast(q, k, q_weight, k_weight, eps, cos, sin, q_out, k_out):
+        status = fast(q, k, q_weight, k_weight, eps, cos, sin, q_out, k_out)
+        if status is True:
             return
         _ndim(4, q=q, k=k, q_out=q_out, k_out=k_out)
         _ndim(1, q_weight=q_weight, k_weight=k_weight)
         _ndim(2, cos=cos, sin=sin)
         device = _bf16(q, k, q_weight, k_weight, cos, sin, q_out, k_out)
-        _lib.launch("launch_h3_qk_norm_rope_interleaved_qk", device, _lib.tensor(q), _lib.tensor(k),
-                    _lib.tensor(q_weight), _lib.tensor(k_weight), _lib.scalar(eps), _lib.tensor(cos),
-                    _lib.tensor(sin), _lib.tensor(q_out), _lib.tensor(k_out))
+        _lib.launch_after(status, "launch_h3_qk_norm_rope_interleaved_qk", device, _lib.tensor(q), _lib.tensor(k),
+                          _lib.tensor(q_weight), _lib.tensor(k_weight), _lib.scalar(eps), _lib.tensor(cos),
+                          _lib.tensor(sin), _lib.tensor(q_out), _lib.tensor(k_out))
 
     return launch
 
@@ -552,7 +577,8 @@ def make_rope_cache(caller="torch", output_dir=None, archs=None, block_tokens=64
     fast = _lib.fast("launch_h3_rope_cache", "d2f1b2b2")
 
     def kernel(position, power, cos, sin):
-        if fast(position, power, cos, sin):
+        status = fast(position, power, cos, sin)
+        if status is True:
             return
         _ndim(2, position=position, cos=cos, sin=sin)
         _ndim(1, power=power)
@@ -560,7 +586,7 @@ def make_rope_cache(caller="torch", output_dir=None, archs=None, block_tokens=64
         _lib.check_dtype(torch.float64, position)
         _lib.check_dtype(torch.float32, power)
         _lib.check_dtype(torch.bfloat16, cos, sin)
-        _lib.launch("launch_h3_rope_cache", device, _lib.tensor(position), _lib.tensor(power),
-                    _lib.tensor(cos), _lib.tensor(sin))
+        _lib.launch_after(status, "launch_h3_rope_cache", device, _lib.tensor(position), _lib.tensor(power),
+                          _lib.tensor(cos), _lib.tensor(sin))
 
     return kernel

@@ -2,7 +2,10 @@
 what it leaves to the checked Python path."""
 from __future__ import annotations
 
+import contextlib
+import ctypes
 import importlib
+import types
 
 import pytest
 import torch
@@ -33,6 +36,102 @@ def test_other_than_plain_cuda_tensors_are_not_taken(native):
     for args in [(x, w), (x, w, 1.0, 2), (x, w, 1.0), (x, 3, 1.0), (None, w, 1.0), (x, w, "a"),
                  (torch.nn.Buffer(x), w, 1.0)]:
         assert native.call(plan, *args) is False
+
+
+# Every factory with a native call, and tensors of its arguments' ranks.
+CALLS = [
+    ("make_swiglu", "x3 x3 x3"), ("make_rms", "x3 x1 e x3", dict(width=None)),
+    ("make_rms_modulate", "x3 x1 e x3 x3 x3"),
+    ("make_gated_residual", "x3 x3 x3 x3"), ("make_gated_residual_rms_modulate", "x3 x3 x3 x1 e x3 x3 x3 x3"),
+    ("make_rms_modulate_indexed", "x3 x1 e x2 x2 i x3", dict(check_indices=False)),
+    ("make_gated_residual_rms_modulate_indexed", "x3 x2 x3 x1 e x2 x2 i x3 x3", dict(check_indices=False)),
+    ("make_gated_residual_indexed", "x3 x2 x3 i x3", dict(check_indices=False)), ("make_rope", "x3 x2 x2 x3"),
+    ("make_qk_norm_rope", "x4 x1 e x2 x2 x4"), ("make_qkv_norm_rope_pack", "x4 x4 x4 x1 x1 e c p x4 x4 x4"),
+    ("make_qkv_norm_rope_pack_fp8", "x4 x4 x4 x1 x1 e c p q q x4 f f"),
+    ("make_qkv_norm_rope_pack_fp8_vamax", "x4 x4 x4 x1 x1 e c p q q x4 f f a"),
+    ("make_qkv_norm_rope_pack_fp8x2_vamax", "x4 x4 x4 x1 x1 e c p q q q q x4 f f a"),
+    ("make_qk_norm_rope_interleaved", "x4 x1 e x2 x2 x4"),
+    ("make_qk_norm_rope_interleaved_qk", "x4 x4 x1 x1 e x2 x2 x4 x4"), ("make_rope_cache", "d2 f x2 x2"),
+    ("make_attention", "x4 x4 x4 e x4"), ("make_attention", "x4 x4 x4 e x4", dict(split_last_round=False)),
+    ("make_attention_fp8", "q q q f f f e x4"), ("make_attention_fp8x2", "q q q q q f f f e x4"),
+    ("make_attention_fp8pv", "x4 x4 q f e x4"), ("quantize_fp8_per_head", "x4 k q f a"),
+]
+
+
+@pytest.mark.parametrize("status", [1, 98, 700])
+@pytest.mark.parametrize("factory,kinds,options", [(c + ({},))[:3] for c in CALLS])
+def test_a_launch_that_returns_an_error_is_not_repeated(pkg, monkeypatch, factory, kinds, options, status):
+    """A launcher's status can be an error an earlier call left, with its kernel
+    queued all the same: it is raised, and the entry point is not called again."""
+    shape = {"1": (128,), "2": (1, 128), "3": (1, 1, 128), "4": (1, 1, 1, 128)}
+    make = {"x": lambda k: torch.zeros(shape[k[1]], dtype=BF), "e": lambda k: EPS,
+            "i": lambda k: torch.zeros(1, 1).long(),
+            "c": lambda k: torch.zeros(1, 96, dtype=BF), "p": lambda k: torch.zeros(1).long(),
+            "q": lambda k: torch.zeros(1, 1, 1, 128, dtype=torch.float8_e4m3fn), "f": lambda k: torch.zeros(1),
+            "a": lambda k: torch.zeros(1, 64), "d": lambda k: torch.zeros(1, 3).double(), "k": lambda k: False}
+    args = [make[k[0]](k) for k in kinds.split()]
+    native, direct = [], []
+    monkeypatch.setattr(pkg._lib, "fast", lambda name, *a, **kw: lambda *args: native.append(name) or status)
+    monkeypatch.setattr(pkg._lib, "call", lambda name, *a: direct.append(name) or 0)
+    monkeypatch.setattr(pkg._lib, "check_cuda", lambda *t: torch.device("cuda:0"))
+    monkeypatch.setattr(pkg._lib, "planned_workspace", lambda *sizes: 0)
+    attention = importlib.import_module("minimaxh3_on_k100-ai_amd.h3_attention")
+    pointwise = importlib.import_module("minimaxh3_on_k100-ai_amd.h3_pointwise")
+    attention._slots_fast.cache_clear()
+    monkeypatch.setattr(pointwise, "_positions", lambda p, device: p)
+    if factory == "make_qkv_norm_rope_pack":  # compares the device of its positions itself
+        monkeypatch.setattr(pkg._lib, "check_cuda", lambda *t: t[0].device)
+    if factory == "make_attention":
+        monkeypatch.setattr(torch, "empty", lambda *a, device=None, **kw: torch.zeros(*a, **kw))
+    fn = getattr(pkg, factory) if factory.startswith("quantize") else getattr(pkg, factory)(**options)
+    try:
+        with pytest.raises(pkg._lib.LaunchError) as e:
+            fn(*args)
+    finally:
+        attention._slots_fast.cache_clear()
+    assert e.value.status == status and len(native) == 1 and direct == []
+
+
+def test_python_path_launches_what_the_native_call_left(pkg, monkeypatch):
+    called = []
+    monkeypatch.setattr(pkg._lib, "call", lambda name, *a: called.append(name) or 0)
+    monkeypatch.setattr(torch.cuda, "device", lambda d: contextlib.nullcontext())
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda d: types.SimpleNamespace(cuda_stream=0))
+    pkg._lib.launch_after(False, "launch_h3_swiglu_exact", torch.device("cuda:0"))
+    assert called == ["launch_h3_swiglu_exact"]
+
+
+@pytest.mark.gpu
+def test_native_call_returns_the_status_of_its_one_launch(pkg, native, device):
+    statuses = [0, 1, 98, 700]
+    calls = []
+    signature = ctypes.CFUNCTYPE(ctypes.c_int, ctypes.c_void_p, *[pkg._lib.NineToothedTensor] * 3)
+    launcher = signature(lambda *a: calls.append(a) or statuses[len(calls) - 1])
+    plan = native.plan(ctypes.cast(launcher, ctypes.c_void_p).value, "b3b3b3", (0, 1, 2), None)
+    x = torch.zeros(1, 2, 8, dtype=BF, device=device)
+    assert [native.call(plan, x, x, x) for _ in statuses] == [True, 1, 98, 700]
+    assert native.call(plan, x, x, x.float()) is False and len(calls) == len(statuses)
+
+
+@pytest.mark.gpu
+def test_an_error_left_by_another_call_is_raised_after_one_launch(pkg, device):
+    """In place, so that a second launch would show: the gated residual reports
+    the thread's earlier error (a device that does not exist) and ran once."""
+    hip = ctypes.CDLL("libamdhip64.so")
+    x = torch.ones(1, 64, 1024, dtype=BF, device=device)
+    kernel = pkg.make_gated_residual()
+    kernel(x.clone(), x, x, x.clone())  # bound
+    torch.cuda.synchronize()
+    one = torch.ones_like(x)
+    torch.cuda.synchronize()
+    assert hip.hipSetDevice(4096) != 0
+    with pytest.raises(pkg._lib.LaunchError):
+        kernel(x, one, one, x)
+    torch.cuda.synchronize()
+    assert torch.equal(x, one * 2)
+    kernel(x, one, one, x)
+    torch.cuda.synchronize()
+    assert torch.equal(x, one * 3)
 
 
 @pytest.mark.gpu
