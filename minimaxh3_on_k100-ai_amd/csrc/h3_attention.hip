@@ -89,6 +89,12 @@ template <int DIM>
 constexpr int dim_blocks() { return (DIM + 31) / 32; }
 __device__ __forceinline__ int swz_v(int row) { return 4 * (row & 3); }
 constexpr float kLog2e = 1.4426950408889634f;
+// A query's maximum before any key: below every finite logit, and finite itself,
+// so that keys at -inf get the weight exp2(-inf - m) = 0 also where every key a
+// tile, piece or key group has taken so far is at -inf (from m = -inf it would
+// be exp2(-inf + inf) = NaN). Queries whose keys are all at -inf still end as
+// 0 / 0 = NaN.
+constexpr float kNoMax = -__FLT_MAX__;
 
 struct AttnArgs {
     const bf16_t *q, *k, *v;
@@ -459,7 +465,7 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
     float l_run[kQS];
 #pragma unroll
     for (int qs = 0; qs < kQS; ++qs) {
-        m_run[qs] = -INFINITY;
+        m_run[qs] = kNoMax;
         l_run[qs] = 0.0f;  // running denominator
     }
 
@@ -759,7 +765,7 @@ __device__ __forceinline__ void pv_tile16(const bf16_t *vt, int vidx, const f32x
 
 // A tile with the running-maximum rescale: the tile's maximum, and when it
 // raises the running maximum m of some query, O and the denominator scaled by
-// exp2(m_old - m_new) first (the reference's order). From m = -inf, l = 0,
+// exp2(m_old - m_new) first (the reference's order). From m = kNoMax, l = 0,
 // O = 0 it sets the reference maximum of the first tile.
 template <bool MASK, bool NEG, int NQB, int KS, int DB>
 __device__ __forceinline__ void exact_tile16(const bf16_t *kt, const bf16_t *vt, int valid,
@@ -1003,7 +1009,7 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
         constexpr int NQ = sizeof(mm) / sizeof(float);
 #pragma unroll
         for (int qb = 0; qb < NQ; ++qb) {
-            mm[qb] = -INFINITY;
+            mm[qb] = kNoMax;
             ll[qb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int db = 0; db < DB; ++db)
@@ -1194,7 +1200,7 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
             constexpr int NQ = sizeof(mm) / sizeof(float);
 #pragma unroll
             for (int qb = 0; qb < NQ; ++qb) {
-                mm[qb] = -INFINITY;
+                mm[qb] = kNoMax;
                 ll[qb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
                 for (int db = 0; db < 8; ++db)
@@ -1395,7 +1401,7 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(2, 2
         constexpr bool EXACT = DIM != kD || decltype(exact_tag)::value;
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb) {
-            m[qb] = -INFINITY;
+            m[qb] = kNoMax;
             l[qb] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
             for (int db = 0; db < DB; ++db) acc[qb][db] = f32x4_t{0.0f, 0.0f, 0.0f, 0.0f};
@@ -1480,7 +1486,7 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(2, 2
         const int query = qbk * kQueries + 64 * half + r;
         if (query >= a.Sq) break;
         float2 st[kGroups];
-        float m_all = -INFINITY;
+        float m_all = kNoMax;
 #pragma unroll
         for (int p = 0; p < kGroups; ++p) {
             st[p] = state[p][64 * half + r];

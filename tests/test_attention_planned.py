@@ -9,7 +9,7 @@ import pytest
 import torch
 
 from conftest import attention_error
-from test_attention_gpu import MAX_ABS, REL_RMS, _bhsd, _dominant_keys
+from test_attention_gpu import MAX_ABS, REL_RMS, _bhsd, _dominant_keys, gpu_reference_fp32
 
 BF = torch.bfloat16
 _BUF = ctypes.create_string_buffer(1 << 16)
@@ -109,3 +109,43 @@ def test_short_units_reference_maximum(pkg, oracle, device, D, case):
         assert torch.equal(got, torch.full_like(got, 1.96875))
     rel = float((got.double() - want).norm() / want.norm())
     assert rel <= REL_RMS, rel
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("sign", [1.0, -1.0])
+@pytest.mark.parametrize("D,B,H,Sq,Sk,planned,kernel,masked", [
+    (128, 1, 1, 256, 256, True, "attention16_short_kernel", (64, 96)),   # the third of four key groups of a tile
+    (128, 1, 1, 256, 256, True, "attention16_short_kernel", (0, 128)),   # every group of the first tile
+    (128, 1, 16, 1537, 300, True, "attention16_short_kernel", (0, 64)),  # the first of two groups
+    (72, 1, 1, 256, 256, True, "attention16_short_kernel", (64, 96)),
+    (72, 1, 16, 1537, 300, True, "attention16_short_kernel", (0, 128)),
+    (128, 1, 1, 256, 6400, True, "attention16_kernel", (0, 3200)),       # whole pieces and the first tile of one
+    (72, 2, 3, 1000, 3001, True, "attention16_kernel", (0, 1600)),
+    (72, 1, 16, 4096, 150, False, "attention16_kernel", (0, 64)),        # a unit's first tile
+    (128, 1, 2, 300, 150, False, "attention16_kernel", (0, 64)),
+    (128, 1, 14, 8192, 150, False, "attention16_small_kernel", (0, 64)),
+    (72, 1, 2, 300, 150, False, "attention_fwd_kernel", (0, 64)),
+])
+def test_keys_at_minus_infinity(pkg, device, sign, D, B, H, Sq, Sk, planned, kernel, masked):
+    """Keys masked through a channel of K at -inf, all that a wave's key group, a
+    workgroup's key piece or a unit takes its first maximum from: their weight
+    is 0, and the result is that of the other keys. With every key masked it is
+    NaN, as a softmax over no keys."""
+    gen = torch.Generator(device).manual_seed(Sk + D)
+    q, k, v = (torch.randn(B, H, s, D, generator=gen, device=device).to(BF) for s in (Sq, Sk, Sk))
+    q[..., 0] = 1.0
+    keep = torch.ones(Sk, dtype=torch.bool, device=device)
+    keep[masked[0]:masked[1]] = False
+    k[:, :, ~keep, 0] = float("-inf") * sign
+    out = torch.full_like(q, 3.0)
+    attn = pkg.make_attention(head_dim=D, split_last_round=planned)
+    names = _kernels(lambda: attn(q, k, v, sign * D ** -0.5, out))
+    if torch.cuda.get_device_properties(device).multi_processor_count == 256:
+        assert kernel + "<" in names[0], names
+    want = gpu_reference_fp32(q, k[:, :, keep].contiguous(), v[:, :, keep].contiguous(), sign * D ** -0.5)
+    assert torch.isfinite(out.float()).all()
+    mx, rel = attention_error(out, want)
+    assert mx <= MAX_ABS and rel <= REL_RMS, (mx, rel)
+    k[..., 0] = float("-inf") * sign
+    attn(q, k, v, sign * D ** -0.5, out)
+    assert torch.isnan(out.float()).all()
