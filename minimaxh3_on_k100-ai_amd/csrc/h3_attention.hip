@@ -1307,6 +1307,21 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
         run(std::integral_constant<int, 2>{});
 }
 
+// The merges' weight exp2(m - m_all) of a partial result, as two factors: a
+// partial kept against a maximum below m_all may hold values up to
+// FLT_MAX / kMaxSplit, and a weight below 2^-126, which one exp2 flushes to
+// zero, still leaves a term of order 1. Above 2^-125 the second factor is 1.
+struct MergeWeight {
+    float a, b;
+    MergeWeight() = default;
+    __device__ __forceinline__ explicit MergeWeight(float d) {
+        const bool one = d >= -125.0f;
+        a = __builtin_amdgcn_exp2f(one ? d : 0.5f * d);
+        b = one ? 1.0f : a;
+    }
+    __device__ __forceinline__ float operator*(float x) const { return a * (b * x); }
+};
+
 // The kernel of launches with few units: 32 QW queries per workgroup (QW = 2
 // or 4), the keys of every 128-key tile split over its waves. Wave w takes the
 // 32 queries w % QW of the unit against key group w / QW of each tile (8 / QW
@@ -1492,11 +1507,12 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(2, 2
             st[p] = state[p][64 * half + r];
             m_all = fmaxf(m_all, st[p].x);
         }
-        float w[kGroups], den = 0.0f;
+        MergeWeight w[kGroups];
+        float den = 0.0f;
 #pragma unroll
         for (int p = 0; p < kGroups; ++p) {
-            w[p] = __builtin_amdgcn_exp2f(st[p].x - m_all);
-            den += st[p].y * w[p];
+            w[p] = MergeWeight(st[p].x - m_all);
+            den += w[p] * st[p].y;
         }
         const float inv = __fdiv_rn(1.0f, den);
         bf16_t *orow = obase + static_cast<int64_t>(query) * a.os[2];
@@ -1524,7 +1540,8 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(2, 2
 // Combines the SPLIT pieces of the tail units: a 256-thread block per (tail
 // unit, 8 queries), a thread per (query, 4 dims), all SPLIT pieces' loads
 // issued together. With M = max_p m_p and w_p = 2^(m_p - M):
-// o = bf16((sum_p w_p acc_p) / (sum_p w_p l_p)), sums in piece order.
+// o = bf16((sum_p w_p acc_p) / (sum_p w_p l_p)), sums in piece order, w_p a
+// MergeWeight.
 template <int SPLIT, int DIM>
 __global__ __launch_bounds__(256) void attention_merge_kernel(AttnArgs a) {
     const int u = static_cast<int>(blockIdx.x) / (kBM / 8);
@@ -1551,8 +1568,8 @@ __global__ __launch_bounds__(256) void attention_merge_kernel(AttnArgs a) {
     float den = 0.0f;
 #pragma unroll
     for (int p = 0; p < SPLIT; ++p) {
-        const float w = __builtin_amdgcn_exp2f(st[p].x - m_all);
-        den += st[p].y * w;
+        const MergeWeight w(st[p].x - m_all);
+        den += w * st[p].y;
         sum.x += w * part[p].x;
         sum.y += w * part[p].y;
         sum.z += w * part[p].z;

@@ -149,3 +149,32 @@ def test_keys_at_minus_infinity(pkg, device, sign, D, B, H, Sq, Sk, planned, ker
     k[..., 0] = float("-inf") * sign
     attn(q, k, v, sign * D ** -0.5, out)
     assert torch.isnan(out.float()).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D", [128, 72])
+@pytest.mark.parametrize("H,Sq,Sk,low", [
+    (1, 256, 700, 333),    # four key groups to a tile: keys 5 and 333 in different ones
+    (16, 1537, 700, 333),  # two
+    (1, 256, 6400, 3400),  # the pieces of a key split
+])
+def test_merge_keeps_keys_far_above_their_own_reference(pkg, oracle, device, D, H, Sq, Sk, low):
+    """Key 5 sits 126.5 log2 units above the zeros and sets its part's reference
+    maximum; key `low`, two units below it, is in a part whose first tile has
+    zeros only. Its weight there (2^124.5) needs no recompute, and the merge has
+    to bring it back by 2^-126.5, below the smallest normal number."""
+    gen = torch.Generator("cpu").manual_seed(Sk)
+    q, k = torch.zeros(1, H, Sq, D), torch.zeros(1, H, Sk, D)
+    v = (torch.rand(1, H, Sk, D, generator=gen) * 2 - 1).to(BF)  # |p v| < 2^125: no recompute for O either
+    q[..., 0] = 16.0
+    k[:, :, 5, 0], k[:, :, low, 0] = 62.0, 61.0  # 126.50 and 124.46 log2 units
+    q, k = q.to(BF), k.to(BF)
+    scale = 128 ** -0.5
+    out = torch.full(q.shape, float("nan"), dtype=BF, device=device)
+    attn = pkg.make_attention(head_dim=D)
+    names = _kernels(lambda: attn(q.to(device), k.to(device), v.to(device), scale, out))
+    if torch.cuda.get_device_properties(device).multi_processor_count == 256:
+        assert ("short" in names[0]) == (Sk == 700) and len(names) == (1 if Sk == 700 else 2), names
+    want = oracle.attention(q[:, :, :1].double(), k.double(), v.double(), scale).expand(q.shape)
+    mx, rel = attention_error(out.cpu(), want)
+    assert mx <= MAX_ABS and rel <= REL_RMS, (mx, rel)
