@@ -88,9 +88,9 @@ NineToothedResult launch_h3_full_attention_ws(NineToothedStream stream, NineToot
 int64_t h3_full_attention_workspace_bytes(int64_t B, int64_t H, int64_t Sq, int64_t Sk);
 
 /* The same operator built for head dim 72 (the Qwen vision tower's heads):
- * q, o: [B, H, Sq, 72]; k, v: [B, H, Sk, 72]; views, masking and numerics as
- * launch_h3_full_attention (views outside its 16-byte tile path take the
- * reference's own order: a running maximum with rescaling, fp32 denominator).
+ * q, o: [B, H, Sq, 72]; k, v: [B, H, Sk, 72]; views and masking as
+ * launch_h3_full_attention, fp32_qk numerics in the reference's own order
+ * (a running maximum with rescaling, fp32 denominator).
  * Returns an error for any other head dim, as launch_h3_full_attention does
  * for a head dim other than 128.
  * Replaces launch_h3_vision_attention_72 (scripts/build_h3_attention.py:23-24,
@@ -102,9 +102,11 @@ NineToothedResult launch_h3_vision_attention_72(NineToothedStream stream, NineTo
                                                 NineToothedTensor scale, NineToothedTensor o);
 
 /* launch_h3_full_attention_ws (head dim 128) or the same for head dim 72, by
- * q's head dim, that may also run a launch of few units as units of 64 queries
- * whose keys are split over the waves of a workgroup (running maximum, no
- * workspace): whichever the shapes make fastest. Results are within the
+ * q's head dim, that may also run a launch of few units as units of 64 or 128
+ * queries whose keys are split over the waves of a workgroup (no workspace):
+ * whichever the shapes make fastest. Each wave, or each piece of the key split,
+ * keeps its own maximum (at head dim 128 its first tile's, with the recompute
+ * of launch_h3_full_attention; at 72 a running one). Results are within the
  * operator's tolerance of the unsplit launch and deterministic. It uses
  * h3_attention_planned_workspace_bytes(B, H, Sq, Sk, D) bytes (0: pass an
  * empty workspace; a smaller one runs without the key split). No counterpart

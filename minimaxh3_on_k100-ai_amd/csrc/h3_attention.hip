@@ -25,11 +25,11 @@
 //     and denominator in the workspace and a merge kernel combines them (the
 //     same algebra as the online rescale).
 //
-// attention16_kernel (the buffer path: the configurations and the vision
-// tower) runs on v_mfma_f32_16x16x32_bf16 and keeps one reference maximum per
+// attention16_kernel (the buffer path at D = 128, the key split at both head
+// dims) runs on v_mfma_f32_16x16x32_bf16 and keeps one reference maximum per
 // unit (its layout and numerics are described above it). attention_fwd_kernel
 // runs on v_mfma_f32_32x32x16_bf16 with the exact online rescale and serves
-// K/V views outside the buffer path and D = 72 launches that leave CUs idle:
+// K/V views outside the buffer path and the unsplit launches of D = 72:
 //
 // MFMA formulation (v_mfma_f32_32x32x16_bf16; A row = lane % 32, B column =
 // lane % 32, accumulator register i of lane l holds row 8*(i/4) + 4*(l/32) + i%4)
@@ -584,7 +584,8 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
 
 // ============================================================ attention16_kernel
 //
-// The kernel of the buffer path, on v_mfma_f32_16x16x32_bf16: under
+// The kernel of the buffer path at D = 128 and of the key split at 72, on
+// v_mfma_f32_16x16x32_bf16: under
 // power the part sustains about 14% more flops with this product than with
 // 32x32x16 (launch_h3_calibration_mfma_16x16x32).
 //
@@ -714,6 +715,7 @@ __device__ __forceinline__ void pv_tile16(const bf16_t *vt, int vidx, const f32x
                     if (16 * kb + 4 * g + i >= valid) e = 0.0f;
                 }
                 p[kb][i] = e;
+                if constexpr (DB != dim_blocks16<kD>()) l[qb][kb & 1] += e;
             }
 #pragma unroll
         for (int h = 0; h < KB / 2; ++h) {
@@ -727,7 +729,8 @@ __device__ __forceinline__ void pv_tile16(const bf16_t *vt, int vidx, const f32x
     }
     // The denominator on the matrix core: ones x P^T adds the 32 keys of each
     // half to every row of l (each lane then holds its query's whole sum). At
-    // D = 72 dim 72 of V is taken as ones, and the sum falls out of P V.
+    // D = 72 it is the fp32 sum of the unrounded weights above, each lane's own
+    // 16 keys of a tile in l[qb][0] + l[qb][1] (folded in den_total).
     if constexpr (DB == dim_blocks16<kD>()) {
         const bf16x8_t ones = as_bf16x8(make_uint4(0x3f803f80u, 0x3f803f80u, 0x3f803f80u, 0x3f803f80u));
 #pragma unroll
@@ -743,12 +746,7 @@ __device__ __forceinline__ void pv_tile16(const bf16_t *vt, int vidx, const f32x
             const i16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t *)(vp));
             const i16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_i16x4_t *)(vp + 16 * kRow));
             const uint2 lo2 = __builtin_bit_cast(uint2, lo), hi2 = __builtin_bit_cast(uint2, hi);
-            uint4 vw = make_uint4(lo2.x, lo2.y, hi2.x, hi2.y);
-            if (DB != dim_blocks16<kD>() && db == DB - 1) {  // dim 72's row: ones over its zeros
-                const uint32_t one = (threadIdx.x & 15) == 8 ? 0x3f803f80u : 0u;
-                vw = make_uint4(vw.x | one, vw.y | one, vw.z | one, vw.w | one);
-            }
-            const bf16x8_t vop = as_bf16x8(vw);
+            const bf16x8_t vop = as_bf16x8(make_uint4(lo2.x, lo2.y, hi2.x, hi2.y));
 #pragma unroll
             for (int qb = 0; qb < NQB; ++qb)
                 acc[qb][db] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vop, pop[qb][h], acc[qb][db], 0, 0, 0);
@@ -857,7 +855,7 @@ __device__ __forceinline__ void running_tile16(const bf16_t *kt, const bf16_t *v
             const float n = mt > m[qb] ? mt : m[qb];
             const float al = __builtin_amdgcn_exp2f(m[qb] - n);
             m[qb] = n;
-            if constexpr (DB == dim_blocks16<kD>()) l[qb] *= al;
+            l[qb] *= al;
 #pragma unroll
             for (int db = 0; db < DB; ++db)
 #pragma unroll
@@ -877,14 +875,19 @@ __device__ __forceinline__ void ref_tile16(const bf16_t *kt, const bf16_t *vt, i
     pv_tile16<MASK>(vt, vidx, s, m, l, c, valid, g, acc);
 }
 
-// A query's denominator: every row of its l accumulator holds the whole sum;
-// at D = 72 it is O^T's row 72, register 0 of dim block 4 in lane group 2.
-template <int DB>
-__device__ __forceinline__ float den_total(const f32x4_t &l, const f32x4_t (&acc)[DB], int l16) {
-    if constexpr (DB == dim_blocks16<kD>())
+// A query's denominator: every row of its l accumulator holds the whole sum; at
+// D = 72 the four lanes of the query hold their own keys' (see pv_tile16).
+template <int DIM>
+__device__ __forceinline__ float den_total(const f32x4_t &l) {
+    if constexpr (DIM == kD) {
         return l[0];
-    else
-        return __shfl(acc[4][0], 32 + l16, 64);
+    } else {
+        float x = l[0] + l[1];
+        const auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        x = __uint_as_float(a[0]) + __uint_as_float(a[1]);
+        const auto b = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(x), false, false);
+        return __uint_as_float(b[0]) + __uint_as_float(b[1]);
+    }
 }
 
 // The Q^T operands of query block qb (k-step ks: dims 32 ks + 8 g .. +8 of
@@ -922,10 +925,11 @@ __device__ __forceinline__ void load_q16(const AttnArgs &a, const bf16_t *qbase,
 // O, reference maximum and denominator in the workspace for the merge.
 // DIM: the head dim, 128 or 72. At 72 the tiles keep the 128-dim row layout
 // (chunks past the head dim are zeros), 3 k-steps and 5 dim blocks hold the 72
-// dims, and dim 72's row of O^T is the denominator: 44 products per tile and
-// wave. It keeps the running maximum: against a fixed one its error against
-// float64 was 2-5% larger than the 32x32x16 kernel's it replaces, with it 1-3%
-// smaller (over S = 256 .. 16,384, N(0, 1) and 1% of key rows x8).
+// dims: 44 products per tile and wave. It keeps the reference's order, as the
+// 32x32x16 kernel of its unsplit launches does: the running maximum (against a
+// fixed one the error against float64 was 2-5% larger) and the fp32 sum of the
+// unrounded weights. Error against float64 over S = 256 .. 16,384, N(0, 1) and
+// 1% of key rows x8: 0.3-5% below the 32x32x16 kernel's.
 template <bool NEG, bool SPLIT, int DIM>
 __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWaves / 4, kWaves / 4))) void attention16_kernel(AttnArgs a) {
     __shared__ __attribute__((aligned(1024))) bf16_t lds_k0[kTileElems];
@@ -1063,7 +1067,7 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
     // its last LDS read of the pass before the barrier.
     float lt[2];
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb) lt[qb] = den_total(l[qb], acc[qb], l16);
+    for (int qb = 0; qb < 2; ++qb) lt[qb] = den_total<DIM>(l[qb]);
     const float limit = piece >= 0 ? __FLT_MAX__ / kMaxSplit : INFINITY;
     // x < limit is false for NaN, so NaN counts as overflow too.
     bool finite = lt[0] < limit && lt[1] < limit;
@@ -1089,7 +1093,7 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
             load_q16(a, qbase, q_first, qb, l16, g, q1[0]);
             pass(std::true_type{}, q1, *reinterpret_cast<float(*)[1]>(&m[qb]), *reinterpret_cast<f32x4_t(*)[1]>(&l[qb]),
                  *reinterpret_cast<f32x4_t(*)[1][DB]>(&acc[qb]));
-            lt[qb] = den_total(l[qb], acc[qb], l16);
+            lt[qb] = den_total<DIM>(l[qb]);
         };
         redo(std::integral_constant<int, 0>{});
         __syncthreads();  // every wave past its last LDS read
@@ -1250,7 +1254,7 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
         // maximum (as attention16_kernel does).
         float lt[NQB];
 #pragma unroll
-        for (int qb = 0; qb < NQB; ++qb) lt[qb] = den_total(l[qb], acc[qb], l16);
+        for (int qb = 0; qb < NQB; ++qb) lt[qb] = den_total<kD>(l[qb]);
         constexpr float limit = INFINITY;
         // x < limit is false for NaN, so NaN counts as overflow too.
         bool finite = true;
@@ -1278,7 +1282,7 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
                 load_q16(a, qbase, q_first, qb, l16, g, q1[0]);
                 pass(std::true_type{}, q1, *reinterpret_cast<float(*)[1]>(&m[qb]),
                      *reinterpret_cast<f32x4_t(*)[1]>(&l[qb]), *reinterpret_cast<f32x4_t(*)[1][8]>(&acc[qb]));
-                lt[qb] = den_total(l[qb], acc[qb], l16);
+                lt[qb] = den_total<kD>(l[qb]);
             };
             redo(std::integral_constant<int, 0>{});
             __syncthreads();  // every wave past its last LDS read
@@ -1336,7 +1340,7 @@ struct MergeWeight {
 // chip, after 7 us of launch, first loads and merge. 14 heads, S = 1024: 14.3
 // against 29.2 us (256-query units split in 2 over workgroups, and the merge
 // launch); S = 256: 9.1 against 14.1 us; S = 2048: 33.1 against 41.8 us; 16 heads
-// of 72, S = 1000: 13.8 against 25.1 us.
+// of 72, S = 1000: 14.4 against 25.1 us.
 constexpr int kShortBN = 128;  // keys per tile
 constexpr int kShortLoads = kShortBN * 16 / kThreadsWG;
 
@@ -1456,7 +1460,7 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(2, 2
         // maximum. The limit leaves room for the sum over the key groups, each
         // weighted by at most 1.
         constexpr float limit = __FLT_MAX__ / kMaxSplit;
-        bool finite = den_total(l[0], acc[0], l16) < limit && den_total(l[1], acc[1], l16) < limit;
+        bool finite = den_total<DIM>(l[0]) < limit && den_total<DIM>(l[1]) < limit;
 #pragma unroll
         for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
@@ -1485,7 +1489,7 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(2, 2
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) {
         const int r = 32 * (qw % 2) + 16 * qb + l16;
-        const float den = den_total(l[qb], acc[qb], l16);
+        const float den = den_total<DIM>(l[qb]);
         if (g == 0) state[kw][32 * qw + 16 * qb + l16] = float2{m[qb], den};
 #pragma unroll
         for (int db = 0; db < DB; ++db)
@@ -1859,17 +1863,15 @@ int launch_attention(NineToothedStream stream, NineToothedTensor q, NineToothedT
                              : launch_split<72>(a, neg, static_cast<unsigned>(plan.n_full + pieces), st);
         }
     }
-    // D = 72 with a fifth or more of the CUs idle: the chip then runs at its top
-    // clock, where the 32x32x16 kernel's tiles take 1.27 us against 1.42 us
-    // (144 to 192 units; 63.3 against 68.9 us at 16 heads, S = 3000), while on a
-    // full chip, under its power limit, the 16x16x32 products win (S = 4096:
-    // 93.3 against 97.3 us; 240 units: 81.9 against 83.4 us).
-    const bool idle72 = dim != kD && 5 * grid <= 4 * static_cast<int64_t>(n_cu);
-    if (buf && !idle72) {
-#define H3_ATTN16(N, D) \
-    if (neg == N && dim == D) attention16_kernel<N, false, D><<<g, kThreadsWG, 0, st>>>(a);
-        H3_ATTN16(false, 128) H3_ATTN16(true, 128) H3_ATTN16(false, 72) H3_ATTN16(true, 72)
-#undef H3_ATTN16
+    // Unsplit launches of D = 72 stay on the 32x32x16 kernel: both carry the same
+    // softmax VALU work, which bounds them, and attention16_kernel's tiles are the
+    // slower ones where CUs idle (16 heads, S = 3400: 75.9 against 81.5 us), level
+    // on a full chip (S = 4096: 95.8 against 97.4; 8192: 366 against 364 us).
+    if (buf && dim == kD) {
+        if (neg)
+            attention16_kernel<true, false, kD><<<g, kThreadsWG, 0, st>>>(a);
+        else
+            attention16_kernel<false, false, kD><<<g, kThreadsWG, 0, st>>>(a);
         return launch_status();
     }
 #define H3_ATTN(N, B, D, G) \

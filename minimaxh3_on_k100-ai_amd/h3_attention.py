@@ -16,13 +16,14 @@ Numerics (tools/h3_attention.py:25-101):
     masked, so the three coincide.
   - "bf16_prescale" (:87-101): q enters the product as bf16(fp32(scale log2 e) q)
     and the logits are used unscaled (launch_h3_full_attention_bf16_prescale).
-  The softmax's stabilising maximum is the first key tile's,
+  At head_dim 128 the softmax's stabilising maximum is the first key tile's,
   kept for the rest of a 256-query unit (the unit is recomputed with the
   running maximum if anything overflows against it), and the denominator
   sums the same bf16-rounded P that multiplies V. The reference rescales at
   every new running maximum and sums P in fp32; the results agree within the
-  operator's tolerance. head_dim 72 takes the same order; K/V views outside
-  the 16-byte tile path keep the reference's.
+  operator's tolerance. head_dim 72, and K/V views outside the 16-byte tile
+  path, keep the reference's order. Where the keys are split (below), each
+  part has its own maximum and the parts are merged in fp32.
 head_dim 128 (the DiT's) and 72 (the Qwen vision tower's, launcher
 launch_h3_vision_attention_72 as in scripts/build_h3_attention.py:23-24) are
 built; as in the reference, a factory runs only tensors of its own head_dim.

@@ -121,10 +121,10 @@ def test_short_units_reference_maximum(pkg, oracle, device, D, case):
     (72, 1, 16, 1537, 300, True, "attention16_short_kernel", (0, 128)),
     (128, 1, 1, 256, 6400, True, "attention16_kernel", (0, 3200)),       # whole pieces and the first tile of one
     (72, 2, 3, 1000, 3001, True, "attention16_kernel", (0, 1600)),
-    (72, 1, 16, 4096, 150, False, "attention16_kernel", (0, 64)),        # a unit's first tile
-    (128, 1, 2, 300, 150, False, "attention16_kernel", (0, 64)),
+    (128, 1, 2, 300, 150, False, "attention16_kernel", (0, 64)),         # a unit's first tile
     (128, 1, 14, 8192, 150, False, "attention16_small_kernel", (0, 64)),
     (72, 1, 2, 300, 150, False, "attention_fwd_kernel", (0, 64)),
+    (72, 1, 16, 4096, 150, False, "attention_fwd_kernel", (0, 64)),
 ])
 def test_keys_at_minus_infinity(pkg, device, sign, D, B, H, Sq, Sk, planned, kernel, masked):
     """Keys masked through a channel of K at -inf, all that a wave's key group, a
@@ -178,3 +178,29 @@ def test_merge_keeps_keys_far_above_their_own_reference(pkg, oracle, device, D, 
     want = oracle.attention(q[:, :, :1].double(), k.double(), v.double(), scale).expand(q.shape)
     mx, rel = attention_error(out.cpu(), want)
     assert mx <= MAX_ABS and rel <= REL_RMS, (mx, rel)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("H,Sq,Sk,kernel", [
+    (1, 256, 704, "attention16_short_kernel<false, 72, 2>"), (16, 1537, 715, "attention16_short_kernel<false, 72, 4>"),
+    (1, 256, 6410, "attention16_kernel<false, true, 72>"), (16, 4096, 705, "attention_fwd_kernel<false, true, 72"),
+])
+def test_vision_denominator_sums_the_unrounded_weights(pkg, device, H, Sq, Sk, kernel):
+    """Head dim 72: the reference's order on every path, bf16 weights on V over
+    the fp32 sum of the weights before that rounding. One key of 16 weighs 1 and
+    the others 0.5019, which rounds to 0.5: V = 1 comes out as (1 + 15 / 2) /
+    (1 + 15 * 0.5019) = 0.9967, not as 1."""
+    q, k = torch.zeros(1, H, Sq, 72), torch.zeros(1, H, Sk, 72)
+    q[..., 0] = 1.0
+    k[:, :, 5::16, 0] = 1.0
+    q, k, v = (t.to(BF).to(device) for t in (q, k, torch.ones(1, H, Sk, 72)))
+    out = torch.full_like(q, float("nan"))
+    attn = pkg.make_attention(head_dim=72)
+    scale = 0.99453 * 0.6931471805599453
+    names = _kernels(lambda: attn(q, k, v, scale, out))
+    if torch.cuda.get_device_properties(device).multi_processor_count == 256:
+        assert kernel in names[0], names
+    weight = 2.0 ** -0.99453
+    high = len(range(5, Sk, 16))
+    want = torch.tensor((high + (Sk - high) * 0.5) / (high + (Sk - high) * weight)).to(BF).item()
+    assert want == 0.99609375 and bool((out == want).all()), out.float().aminmax()
