@@ -1059,45 +1059,47 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
         }
     };
     pass(std::false_type{}, qreg, m, l, acc);
-    // Overflow against the reference maxima: redo the unit with the running
-    // maximum. The test covers the denominator (finite weights can sum to
-    // +inf) and every accumulator. A key piece is held to
-    // FLT_MAX / kMaxSplit, so that the merge's sums over up to kMaxSplit
-    // pieces, each weighted by at most 1, stay finite. Every wave has passed
-    // its last LDS read of the pass before the barrier.
     float lt[2];
 #pragma unroll
     for (int qb = 0; qb < 2; ++qb) lt[qb] = den_total<DIM>(l[qb]);
-    const float limit = piece >= 0 ? __FLT_MAX__ / kMaxSplit : INFINITY;
-    // x < limit is false for NaN, so NaN counts as overflow too.
-    bool finite = lt[0] < limit && lt[1] < limit;
+    if constexpr (DIM == kD) {
+        // Overflow against the reference maxima: redo the unit with the running
+        // maximum. The test covers the denominator (finite weights can sum to
+        // +inf) and every accumulator. A key piece is held to
+        // FLT_MAX / kMaxSplit, so that the merge's sums over up to kMaxSplit
+        // pieces, each weighted by at most 1, stay finite. Every wave has passed
+        // its last LDS read of the pass before the barrier.
+        const float limit = piece >= 0 ? __FLT_MAX__ / kMaxSplit : INFINITY;
+        // x < limit is false for NaN, so NaN counts as overflow too.
+        bool finite = lt[0] < limit && lt[1] < limit;
 #pragma unroll
-    for (int qb = 0; qb < 2; ++qb)
+        for (int qb = 0; qb < 2; ++qb)
 #pragma unroll
-        for (int db = 0; db < DB; ++db)
+            for (int db = 0; db < DB; ++db)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) finite = finite && fabsf(acc[qb][db][i]) < limit;
-    const bool wave_bad = __builtin_amdgcn_ballot_w64(!finite) != 0;
-    if (lane == 0) wave_overflow[wave] = wave_bad ? 1 : 0;
-    __syncthreads();
-    int any_bad = 0;
+                for (int i = 0; i < 4; ++i) finite = finite && fabsf(acc[qb][db][i]) < limit;
+        const bool wave_bad = __builtin_amdgcn_ballot_w64(!finite) != 0;
+        if (lane == 0) wave_overflow[wave] = wave_bad ? 1 : 0;
+        __syncthreads();
+        int any_bad = 0;
 #pragma unroll
-    for (int w = 0; w < kWaves; ++w) any_bad |= wave_overflow[w];
-    if (any_bad) {
-        // The fallback takes one query block at a time, with its Q operands
-        // loaded again, so that it holds half the state of the pass above
-        // (the kernel's register peak otherwise).
-        auto redo = [&](auto qb_tag) __attribute__((always_inline)) {
-            constexpr int qb = decltype(qb_tag)::value;
-            bf16x8_t q1[1][KS];
-            load_q16(a, qbase, q_first, qb, l16, g, q1[0]);
-            pass(std::true_type{}, q1, *reinterpret_cast<float(*)[1]>(&m[qb]), *reinterpret_cast<f32x4_t(*)[1]>(&l[qb]),
-                 *reinterpret_cast<f32x4_t(*)[1][DB]>(&acc[qb]));
-            lt[qb] = den_total<DIM>(l[qb]);
-        };
-        redo(std::integral_constant<int, 0>{});
-        __syncthreads();  // every wave past its last LDS read
-        redo(std::integral_constant<int, 1>{});
+        for (int w = 0; w < kWaves; ++w) any_bad |= wave_overflow[w];
+        if (any_bad) {
+            // The fallback takes one query block at a time, with its Q operands
+            // loaded again, so that it holds half the state of the pass above
+            // (the kernel's register peak otherwise).
+            auto redo = [&](auto qb_tag) __attribute__((always_inline)) {
+                constexpr int qb = decltype(qb_tag)::value;
+                bf16x8_t q1[1][KS];
+                load_q16(a, qbase, q_first, qb, l16, g, q1[0]);
+                pass(std::true_type{}, q1, *reinterpret_cast<float(*)[1]>(&m[qb]), *reinterpret_cast<f32x4_t(*)[1]>(&l[qb]),
+                     *reinterpret_cast<f32x4_t(*)[1][DB]>(&acc[qb]));
+                lt[qb] = den_total<DIM>(l[qb]);
+            };
+            redo(std::integral_constant<int, 0>{});
+            __syncthreads();  // every wave past its last LDS read
+            redo(std::integral_constant<int, 1>{});
+        }
     }
     if constexpr (SPLIT) {
         if (piece >= 0) {  // a piece: O, m and l of its 256 queries go to the workspace
