@@ -761,71 +761,12 @@ __device__ __forceinline__ void pv_tile16(const bf16_t *vt, int vidx, const f32x
     __builtin_amdgcn_sched_group_barrier(0x008, 2 * NQB, 0);
 }
 
-// A tile with the running-maximum rescale: the tile's maximum, and when it
-// raises the running maximum m of some query, O and the denominator scaled by
-// exp2(m_old - m_new) first (the reference's order). From m = kNoMax, l = 0,
-// O = 0 it sets the reference maximum of the first tile.
-template <bool MASK, bool NEG, int NQB, int KS, int DB>
-__device__ __forceinline__ void exact_tile16(const bf16_t *kt, const bf16_t *vt, int valid,
-                                             const bf16x8_t (&qreg)[NQB][KS], int kidx, int vidx, int g, float c,
-                                             float (&m)[NQB], f32x4_t (&l)[NQB], f32x4_t (&acc)[NQB][DB]) {
-    static_assert(NQB == 1 || NQB == 2, "one or two query blocks per wave");
-    f32x4_t s[NQB][4];
-    qk_tile16(kt, qreg, kidx, s);
-    float mt[NQB];
-#pragma unroll
-    for (int qb = 0; qb < NQB; ++qb) {
-        if constexpr (MASK) {
-#pragma unroll
-            for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-                    if (16 * kb + 4 * g + i >= valid) s[qb][kb][i] = NEG ? INFINITY : -INFINITY;
-        }
-        float mx = s[qb][0][0];
-#pragma unroll
-        for (int kb = 0; kb < 4; ++kb)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) mx = NEG ? fminf(mx, s[qb][kb][i]) : fmaxf(mx, s[qb][kb][i]);
-        mt[qb] = fold_groups_max<NEG>(mx) * c;
-    }
-    if constexpr (NQB == 2) {
-        const bool grow0 = mt[0] > m[0], grow1 = mt[1] > m[1];
-        if (__builtin_amdgcn_ballot_w64(grow0 || grow1)) {
-            const float n0 = grow0 ? mt[0] : m[0], n1 = grow1 ? mt[1] : m[1];
-            const float a0 = __builtin_amdgcn_exp2f(m[0] - n0), a1 = __builtin_amdgcn_exp2f(m[1] - n1);
-            m[0] = n0;
-            m[1] = n1;
-            l[0] *= a0;
-            l[1] *= a1;
-#pragma unroll
-            for (int db = 0; db < DB; ++db)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    acc[0][db][i] *= a0;
-                    acc[1][db][i] *= a1;
-                }
-        }
-    } else {
-        const bool grow0 = mt[0] > m[0];
-        if (__builtin_amdgcn_ballot_w64(grow0)) {
-            const float n0 = grow0 ? mt[0] : m[0];
-            const float a0 = __builtin_amdgcn_exp2f(m[0] - n0);
-            m[0] = n0;
-            l[0] *= a0;
-#pragma unroll
-            for (int db = 0; db < DB; ++db)
-#pragma unroll
-                for (int i = 0; i < 4; ++i) acc[0][db][i] *= a0;
-        }
-    }
-    pv_tile16<MASK>(vt, vidx, s, m, l, c, valid, g, acc);
-}
-
-// exact_tile16 with a query block's O rescaled only when one of its own
-// queries' maxima grows, and the cross-lane fold of the maxima run only then:
-// some lane's own maximum exceeds the running one exactly when the folded one
-// does.
+// A tile with the running-maximum rescale: the tile's maximum, and where it
+// raises the running maximum m of one of a query block's queries, that block's O
+// and denominator scaled by exp2(m_old - m_new) first (the reference's order).
+// From m = kNoMax, l = 0, O = 0 it sets the reference maximum of the first tile.
+// The cross-lane fold of the maxima runs only then: some lane's own maximum
+// exceeds the running one exactly when the folded one does.
 template <bool MASK, bool NEG, int KB, int NQB, int KS, int DB>
 __device__ __forceinline__ void running_tile16(const bf16_t *kt, const bf16_t *vt, int valid,
                                                const bf16x8_t (&qreg)[NQB][KS], int kidx, int vidx, int g, float c,
@@ -1224,7 +1165,7 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
                 dma_tile(krs, kvoff, (tile + 1) * kstep, kn);
                 dma_tile(vrs, vvoff, (tile + 1) * vstep, vn);
                 if constexpr (EXACT || decltype(first_tag)::value)
-                    exact_tile16<false, NEG>(kc, vc, kBN, qq, kidx, vidx, g, c, mm, ll, aa);
+                    running_tile16<false, NEG, 4>(kc, vc, kBN, qq, kidx, vidx, g, c, mm, ll, aa);
                 else
                     ref_tile16<false, 4>(kc, vc, kBN, qq, kidx, vidx, g, c, mm, ll, aa);
                 asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
@@ -1243,12 +1184,12 @@ __global__ __launch_bounds__(kThreadsWG) __attribute__((amdgpu_waves_per_eu(kWav
                     const bf16_t *kc = odd ? lds_k1 : lds_k0;
                     const bf16_t *vc = odd ? lds_v1 : lds_v0;
                     if constexpr (EXACT)
-                        exact_tile16<true, NEG>(kc, vc, valid_last, qq, kidx, vidx, g, c, mm, ll, aa);
+                        running_tile16<true, NEG, 4>(kc, vc, valid_last, qq, kidx, vidx, g, c, mm, ll, aa);
                     else
                         ref_tile16<true, 4>(kc, vc, valid_last, qq, kidx, vidx, g, c, mm, ll, aa);
                 }
             } else if (partial) {  // the partial tile is the only one
-                exact_tile16<true, NEG>(lds_k0, lds_v0, valid_last, qq, kidx, vidx, g, c, mm, ll, aa);
+                running_tile16<true, NEG, 4>(lds_k0, lds_v0, valid_last, qq, kidx, vidx, g, c, mm, ll, aa);
             }
         };
         pass(std::false_type{}, qreg, m, l, acc);
