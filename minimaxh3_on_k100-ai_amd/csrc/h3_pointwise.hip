@@ -674,9 +674,12 @@ __global__ __launch_bounds__(kThreads) void rms_stream_kernel(RmsArgs a) {
 // [64, 5376] 3.6 against 10.2 us, [1000, 7168] 9.7 against 14.1 us; the gated op
 // 4.9 against 7.2 us at [256, 5376] and, with per-token rows, 48.4 against 54.9
 // us at [5726, 5376] and 86.8 against 92.8 us at [8192, 7168].
+// A launch holds fewer than 2^32 threads along x (past them it runs only part of
+// its blocks, with no error), so it takes at most kRowBlocks rows from row0 on.
+constexpr int64_t kRowBlocks = int64_t{1} << 23;
 template <int VPT, int MODE>
-__global__ __launch_bounds__(kThreads) void rms_row_kernel(RmsArgs a) {
-    const uint32_t row = blockIdx.x;  // rows < 2^31
+__global__ __launch_bounds__(kThreads) void rms_row_kernel(RmsArgs a, uint32_t row0) {
+    const uint32_t row = row0 + blockIdx.x;  // rows < 2^31
     const uint32_t b = fast_div(row, a.by_s), s = row - b * static_cast<uint32_t>(a.S);
     int64_t mb, ms;
     mod_coords(a.index, b, s, mb, ms);
@@ -829,12 +832,15 @@ int launch_rms_vec(const RmsArgs &a, hipStream_t stream) {
     }
     if constexpr (VEC) {
         if (rows_by_block<MODE>(a, W8)) {
-            const unsigned grid = static_cast<unsigned>(a.rows);
-            switch ((W8 + kThreads - 1) / kThreads) {
-                case 1: rms_row_kernel<1, MODE><<<grid, kThreads, 0, stream>>>(a); break;
-                case 2: rms_row_kernel<2, MODE><<<grid, kThreads, 0, stream>>>(a); break;
-                case 3: rms_row_kernel<3, MODE><<<grid, kThreads, 0, stream>>>(a); break;
-                default: rms_row_kernel<4, MODE><<<grid, kThreads, 0, stream>>>(a); break;
+            for (int64_t row = 0; row < a.rows; row += kRowBlocks) {
+                const unsigned grid = static_cast<unsigned>(a.rows - row < kRowBlocks ? a.rows - row : kRowBlocks);
+                const uint32_t row0 = static_cast<uint32_t>(row);
+                switch ((W8 + kThreads - 1) / kThreads) {
+                    case 1: rms_row_kernel<1, MODE><<<grid, kThreads, 0, stream>>>(a, row0); break;
+                    case 2: rms_row_kernel<2, MODE><<<grid, kThreads, 0, stream>>>(a, row0); break;
+                    case 3: rms_row_kernel<3, MODE><<<grid, kThreads, 0, stream>>>(a, row0); break;
+                    default: rms_row_kernel<4, MODE><<<grid, kThreads, 0, stream>>>(a, row0); break;
+                }
             }
             return launch_status();
         }

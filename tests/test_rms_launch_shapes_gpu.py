@@ -65,3 +65,37 @@ def test_rms_family_launch_shapes_bitwise(pkg, oracle, device, rows, W, mods):
             "norm": want_norm, "plain": oracle.rms_norm(pick(x), w, EPS)}
     for name, got in zip(("mod", "res", "norm", "plain"), outs):
         assert torch.equal(pick(got.cpu()), want[name]), name
+
+
+def test_rms_row_kernel_past_the_x_extent_of_a_grid(pkg, device):
+    """2^24 rows and more, one block of 256 threads each, are more than the
+    2^32 - 1 threads a launch holds along x. The batch is broadcast (stride 0),
+    so that only the outputs take memory: every batch entry is the first one's
+    bits, which a small launch gives as well."""
+    B, S, W, R = 4097, 4099, 520, 5
+    assert B * S > 1 << 24
+    if torch.cuda.mem_get_info(device)[0] < 48 << 30:
+        pytest.skip("48 GiB of device memory needed")
+    gen = torch.Generator("cpu").manual_seed(11)
+    x, y, scale, shift = (_randn(gen, 1, S, W).to(device) for _ in range(4))
+    w, tables = _randn(gen, W).to(device), [_randn(gen, R, W).to(device) for _ in range(3)]
+    index = torch.randint(0, R, (1, S), generator=gen).to(device)
+    big = lambda t: t.expand(B, *t.shape[1:])
+
+    def check(got, want):
+        for b in range(0, B, 256):
+            part = got[b:b + 256]
+            assert bool((part == want).all()), b
+
+    out, small = torch.zeros(B, S, W, dtype=BF, device=device), torch.zeros(1, S, W, dtype=BF, device=device)
+    rms = pkg.make_rms_modulate()
+    rms(x, w, EPS, scale, shift, small)
+    rms(big(x), w, EPS, big(scale), big(shift), out)  # per-row modulation views
+    check(out, small)
+    gated = pkg.make_gated_residual_rms_modulate_indexed(check_indices=False)
+    res, small_res = torch.zeros_like(out), torch.zeros_like(small)
+    gated(x, tables[0], y, w, EPS, tables[1], tables[2], index, small_res, small)
+    out.zero_()
+    gated(big(x), tables[0], big(y), w, EPS, tables[1], tables[2], big(index), res, out)
+    check(res, small_res)
+    check(out, small)
