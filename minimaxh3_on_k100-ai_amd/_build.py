@@ -60,6 +60,7 @@ def _build_call_module() -> Path:
     lib_dir = Path(torch.__file__).resolve().parent / "lib"
     cmd = [os.environ.get("CXX") or "g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-Wall", "-fvisibility=hidden",
            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+           f'-DH3_TORCH_VERSION="{torch.__version__}"',
            *(f"-isystem{p}" for p in cpp_extension.include_paths()), f"-isystem{sysconfig.get_paths()['include']}",
            str(CSRC / "h3_call.cpp"), f"-L{lib_dir}", "-lc10", "-ltorch_cpu", "-ltorch_python",
            f"-Wl,-rpath,{lib_dir}", "-o", str(tmp)]

@@ -15,6 +15,7 @@ from __future__ import annotations
 import ctypes
 import functools
 import importlib
+import warnings
 from pathlib import Path
 from typing import Sequence
 
@@ -121,6 +122,25 @@ def _not_taken(*args) -> bool:
     return False
 
 
+@functools.lru_cache(maxsize=None)
+def _call_module():
+    """The native module, or None where it is missing, does not load or was built
+    against another torch (it reads tensors through that torch's headers): every
+    call then goes through ctypes, with the same kernels and about 10 to 30 us
+    more host time."""
+    try:
+        native = importlib.import_module(__package__ + "._h3call")
+    except ImportError as e:
+        reason = str(e)
+    else:
+        if native.torch_version == torch.__version__:
+            return native
+        reason = f"built against torch {native.torch_version}, running {torch.__version__}"
+    warnings.warn(f"_h3call.so is not used ({reason}): calls go through ctypes. __graft_entry__.build() builds it.",
+                  RuntimeWarning, stacklevel=3)
+    return None
+
+
 def fast(name: str, kinds: str, order: tuple | None = None, fix: tuple | None = None):
     """A callable that calls entry point `name` once when every argument is as
     `kinds` says (csrc/h3_call.cpp: a kind and a rank per argument) and returns
@@ -129,16 +149,15 @@ def fast(name: str, kinds: str, order: tuple | None = None, fix: tuple | None = 
     `launch_after`, which raises a status and launches after False. order: the launcher's
     arguments by index of the call's; fix: (argument, dim, size) that must hold.
     Without the library it takes no call, and the ctypes path raises at first
-    use."""
+    use; without the native module it takes none, and the ctypes path launches."""
     key = (name, kinds, order, fix)
     bound = _fast_calls.get(key)
     if bound is None:
         if not LIBRARY_PATH.exists():
             return _not_taken
-        try:
-            native = importlib.import_module(__package__ + "._h3call")
-        except ImportError as e:
-            raise ImportError("_h3call.so is missing or does not load: build it with __graft_entry__.build()") from e
+        native = _call_module()
+        if native is None:
+            return _not_taken
         address = ctypes.cast(getattr(library(), name), ctypes.c_void_p).value
         order = tuple(range(len(kinds) // 2)) if order is None else order
         bound = _fast_calls[key] = functools.partial(native.call, native.plan(address, kinds, order, fix))

@@ -254,5 +254,10 @@ PyMODINIT_FUNC PyInit__h3call() {
     get_raw_stream = PyObject_GetAttrString(c, "_cuda_getCurrentRawStream");
     Py_DECREF(c);
     if (get_device == nullptr || get_raw_stream == nullptr) return nullptr;
-    return PyModule_Create(&module);
+    PyObject *m = PyModule_Create(&module);
+    if (m != nullptr && PyModule_AddStringConstant(m, "torch_version", H3_TORCH_VERSION) < 0) {
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
 }

@@ -38,6 +38,38 @@ def test_other_than_plain_cuda_tensors_are_not_taken(native):
         assert native.call(plan, *args) is False
 
 
+@pytest.mark.parametrize("case", ["missing", "does not load", "another torch"])
+def test_factories_work_without_the_native_module(pkg, monkeypatch, case):
+    """With the library there and the native module not usable, factories are
+    made as before it existed, with one warning, and call through ctypes."""
+    name = "minimaxh3_on_k100-ai_amd._h3call"
+    real = importlib.import_module
+
+    def no_module(module, *a):
+        if module != name:
+            return real(module, *a)
+        if case == "another torch":
+            return types.SimpleNamespace(torch_version="0.0.1", plan=None, call=None)
+        raise ImportError("undefined symbol" if case == "does not load" else f"No module named {name!r}")
+
+    called = []
+    monkeypatch.setattr(pkg._lib.importlib, "import_module", no_module)
+    monkeypatch.setattr(pkg._lib, "_fast_calls", {})
+    monkeypatch.setattr(pkg._lib, "LIBRARY_PATH", pkg._lib.Path(__file__))  # there
+    monkeypatch.setattr(pkg._lib, "launch", lambda name, *a: called.append(name))
+    monkeypatch.setattr(pkg._lib, "check_cuda", lambda *t: torch.device("cuda:0"))
+    pkg._lib._call_module.cache_clear()
+    try:
+        with pytest.warns(RuntimeWarning, match="_h3call") as warned:
+            swiglu, _ = pkg.make_swiglu(), pkg.make_attention()
+        assert len(warned) == 1
+        x = torch.zeros(1, 2, 8, dtype=BF)
+        swiglu(x, x, x)
+    finally:
+        pkg._lib._call_module.cache_clear()
+    assert called == ["launch_h3_swiglu_exact"]
+
+
 # Every factory with a native call, and tensors of its arguments' ranks.
 CALLS = [
     ("make_swiglu", "x3 x3 x3"), ("make_rms", "x3 x1 e x3", dict(width=None)),
