@@ -18,14 +18,14 @@ def _randn(gen, *shape, scale=1.0, mean=0.0):
 # One launch per side of every bound: 1536 rows, 2048 / 3072 rows of W8 > 512,
 # 8192 gated rows; W8 = 65 (one group past a wave), 512 / 513, 672 (a half last
 # wave group), 768 and 1024 (exact), 1023.
-@pytest.mark.parametrize("rows,W", [
-    (1535, 520), (1536, 520), (1536, 4096), (1537, 4104), (2048, 5376), (2049, 5376), (3072, 8184), (3073, 8192),
-    (1600, 6144), (8191, 5376), (8192, 5376),
-])
-@pytest.mark.parametrize("mods", ["broadcast", "per_token", "per_row"])
+SIZES = [(1535, 520), (1536, 520), (1536, 4096), (1537, 4104), (2048, 5376), (2049, 5376), (3072, 8184), (3073, 8192),
+         (1600, 6144), (8191, 5376), (8192, 5376)]
+
+
+# Per-row views take one launch shape whatever the size.
+@pytest.mark.parametrize("rows,W,mods", [(*s, m) for s in SIZES for m in ("broadcast", "per_token")] +
+                         [(1537, 4104, "per_row"), (2049, 5376, "per_row")])
 def test_rms_family_launch_shapes_bitwise(pkg, oracle, device, rows, W, mods):
-    if mods == "per_row" and rows not in (1537, 2049):
-        pytest.skip("per-row views take one launch shape")
     gen = torch.Generator("cpu").manual_seed(rows + W)
     R = 3
     B, S = (3, rows // 3) if rows % 3 == 0 else (1, rows)
@@ -99,3 +99,38 @@ def test_rms_row_kernel_past_the_x_extent_of_a_grid(pkg, device):
     gated(big(x), tables[0], big(y), w, EPS, tables[1], tables[2], big(index), res, out)
     check(res, small_res)
     check(out, small)
+
+
+@pytest.mark.parametrize("rows,W", [(64, 5376), (2000, 5376), (5726, 5376), (9000, 3072)])
+def test_outputs_in_place_of_inputs(pkg, device, rows, W):
+    """Outputs over the inputs they replace (RMSNorm into x, the residual into x
+    and the norm into y, RoPE and the SwiGLU product into their inputs): the bits
+    of separate outputs, on the one-row-per-block and the persistent launches."""
+    gen = torch.Generator("cpu").manual_seed(rows)
+    x, y = (_randn(gen, 1, rows, W).to(device) for _ in range(2))
+    w = _randn(gen, W, scale=0.1, mean=1.0).to(device)
+    table = [_randn(gen, 3, W, scale=0.1).to(device) for _ in range(3)]
+    index = (torch.arange(rows, device=device) * 3 // rows).view(1, rows)
+    gate, scale, shift = (t[:1].unsqueeze(0).expand(1, rows, W) for t in table)
+    new = lambda: torch.zeros_like(x)
+    rms, mod, gated = pkg.make_rms(width=None), pkg.make_rms_modulate(), pkg.make_gated_residual_rms_modulate()
+    imod, igated = pkg.make_rms_modulate_indexed(False), pkg.make_gated_residual_rms_modulate_indexed(False)
+    ops = [(lambda x, y, r, o: rms(x, w, EPS, o), "x"), (lambda x, y, r, o: mod(x, w, EPS, scale, shift, o), "x"),
+           (lambda x, y, r, o: imod(x, w, EPS, table[1], table[2], index, o), "x"),
+           (lambda x, y, r, o: gated(x, gate, y, w, EPS, scale, shift, r, o), "xy"),
+           (lambda x, y, r, o: igated(x, table[0], y, w, EPS, table[1], table[2], index, r, o), "xy"),
+           (lambda x, y, r, o: pkg.make_swiglu()(x, y, o), "x")]
+    for op, over in ops:
+        r, o, xi, yi = new(), new(), x.clone(), y.clone()
+        op(x, y, r, o)
+        op(xi, yi, xi, yi if over == "xy" else xi)
+        if over == "xy":
+            assert torch.equal(xi, r) and torch.equal(yi, o)
+        else:
+            assert torch.equal(xi, o)
+    heads = x.view(rows, W // 128, 128)
+    cos, sin = (_randn(gen, rows, 48).to(device) for _ in range(2))
+    o, xi = torch.zeros_like(heads), heads.clone()
+    pkg.make_rope()(heads, cos, sin, o)
+    pkg.make_rope()(xi, cos, sin, xi)
+    assert torch.equal(xi, o)

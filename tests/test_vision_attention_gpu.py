@@ -1,7 +1,8 @@
-"""Head dim 72 on the buffer path (attention16_kernel): the padding of the
-72-dim rows, the denominator taken from V's padding dim, the key split of a
-partly filled last round and the overflow fallback, against the fp32 / fp64
-references of the operator."""
+"""Head dim 72 on the buffer path: the padding of the 72-dim rows and the
+running maximum on each of its kernels -- unsplit launches (attention_fwd_kernel),
+the key split of a partly filled last round (attention16_kernel) and the short
+launches (attention16_short_kernel) -- against the fp32 / fp64 references of the
+operator."""
 from __future__ import annotations
 
 import pytest
@@ -9,10 +10,21 @@ import torch
 
 from conftest import attention_error
 from test_attention_gpu import MAX_ABS, REL_RMS, _bhsd, gpu_reference_fp32
+from test_attention_planned import _kernels
 
 pytestmark = pytest.mark.gpu
 BF = torch.bfloat16
 D = 72
+
+
+FWD, SPLIT = "attention_fwd_kernel<{}, true, 72, false>", "attention16_kernel<{}, true, 72>"
+
+
+def _assert_kernel(device, names, kernel, negative):
+    """The launch ran `kernel` (the plans are those of 256 CUs)."""
+    if torch.cuda.get_device_properties(device).multi_processor_count == 256:
+        assert kernel.format("true" if negative else "false") in names[0], names
+        assert len(names) == (2 if kernel == SPLIT else 1), names  # the split's merge
 
 
 @pytest.mark.parametrize("B,H,Sq,Sk,sign,split", [
@@ -21,6 +33,9 @@ D = 72
     (1, 2, 255, 64, 1.0, False),       # one whole key tile
     (1, 2, 257, 65, -1.0, False),      # one key past it
     (1, 1, 16, 63, 1.0, False),        # a partial tile only
+    (1, 16, 3501, 3501, -1.0, False),  # 224 units: ragged queries and keys, negative scale
+    (1, 16, 4000, 63, 1.0, False),     # a nearly full chip with a partial tile only
+    (3, 16, 1280, 1024, 1.0, False),   # whole tiles, several batch entries
 ])
 def test_vision_attention_plans(pkg, device, B, H, Sq, Sk, sign, split):
     """Every plan at its edges, in a fused projection whose neighbours are NaN
@@ -38,7 +53,8 @@ def test_vision_attention_plans(pkg, device, B, H, Sq, Sk, sign, split):
     out = torch.full((B, Sq, H, D), float("nan"), dtype=BF, device=device)
     out2 = torch.full_like(out, float("nan"))
     attn = pkg.make_attention(head_dim=D)
-    attn(q, k, v, sign * D ** -0.5, _bhsd(out))
+    names = _kernels(lambda: attn(q, k, v, sign * D ** -0.5, _bhsd(out)))
+    _assert_kernel(device, names, SPLIT if split else FWD, sign < 0)
     attn(q, k, v * 2, sign * D ** -0.5, _bhsd(out2))
     torch.cuda.synchronize()
     mx, rel = attention_error(_bhsd(out), gpu_reference_fp32(q, k, v, sign * D ** -0.5))
@@ -46,16 +62,17 @@ def test_vision_attention_plans(pkg, device, B, H, Sq, Sk, sign, split):
     assert torch.equal(out2, out * 2)
 
 
+@pytest.mark.parametrize("Sk,planned,kernel", [
+    (700, True, "attention16_short_kernel<{}, 72, 2>"), (6400, True, SPLIT), (700, False, FWD)])
 @pytest.mark.parametrize("case", ["dominated", "late_logit", "denominator", "huge_values"])
-def test_vision_attention_reference_maximum(pkg, oracle, device, case):
-    """A later key far above the first tile's maximum: its V row comes out
-    exactly where it dominates; where p, the denominator (finite weights that
-    sum past FLT_MAX) or O overflows, the unit is recomputed with the running
-    maximum."""
+def test_vision_attention_running_maximum(pkg, oracle, device, case, Sk, planned, kernel):
+    """A later key far above the first tile's maximum raises the running one: its
+    V row comes out exactly where it dominates, and nothing overflows where
+    weights against the first tile's maximum, their sum or O would."""
     gen = torch.Generator("cpu").manual_seed(9)
     q = torch.zeros(1, 1, 300, D)
-    k = torch.zeros(1, 1, 700, D)
-    v = torch.randn(1, 1, 700, D, generator=gen)
+    k = torch.zeros(1, 1, Sk, D)
+    v = torch.randn(1, 1, Sk, D, generator=gen)
     q[..., 0] = 16.0
     scale = 0.1803369  # times log2 e: 0.2601710
     if case == "dominated":
@@ -72,8 +89,9 @@ def test_vision_attention_reference_maximum(pkg, oracle, device, case):
     q, k, v = (t.to(BF) for t in (q, k, v))
     want = oracle.attention(q.double(), k.double(), v.double(), scale)
     out = torch.full(q.shape, float("nan"), dtype=BF, device=device)
-    pkg.make_attention(head_dim=D)(q.to(device), k.to(device), v.to(device), scale, out)
-    torch.cuda.synchronize()
+    attn = pkg.make_attention(head_dim=D, split_last_round=planned)
+    names = _kernels(lambda: attn(q.to(device), k.to(device), v.to(device), scale, out))
+    _assert_kernel(device, names, kernel, False)
     got = out.cpu()
     assert torch.isfinite(got.float()).all()
     if case == "dominated":
