@@ -1280,10 +1280,10 @@ struct MergeWeight {
 // LDS, over the tile buffers, with the merge kernel's algebra: no workspace, no
 // second launch. What bounds it is latency: a tile step takes 1.1 us (QW = 2) or
 // 1.58 us (QW = 4), the rate of attention16_kernel's steps for its share of the
-// chip, after 7 us of launch, first loads and merge. 14 heads, S = 1024: 14.3
+// chip, after 7 us of launch, first loads and merge. 14 heads, S = 1024: 15.1
 // against 29.2 us (256-query units split in 2 over workgroups, and the merge
-// launch); S = 256: 9.1 against 14.1 us; S = 2048: 33.1 against 41.8 us; 16 heads
-// of 72, S = 1000: 14.4 against 25.1 us.
+// launch); S = 256: 9.1 against 14.1 us; S = 2048: 34.2 against 42.5 us; 16 heads
+// of 72, S = 1000: 14.4 against 25.0 us.
 constexpr int kShortBN = 128;  // keys per tile
 constexpr int kShortLoads = kShortBN * 16 / kThreadsWG;
 
@@ -1568,7 +1568,11 @@ namespace {
 // replaces that round by rounds of ceil(T / s) tiles (at least 8 per piece),
 // plus the merge (130 KiB of partials per piece read back at ~3.5 TB/s and
 // ~5 us of launch and latency, against ~1.8 us per tile-step). The split is
-// taken when the model saves at least 3%.
+// taken when the model saves at least 3%. D = 72 is planned with the same
+// constants, although its tile-step takes about 1.5 us and the unsplit launch runs
+// on the 32x32x16 kernel: planned against unsplit at 16 heads, 2100 to 12,500
+// tokens, it is never slower (S = 4200 117 against 169 us, 6250 249 against 255,
+// 6750 and 7250 unsplit, 9500 513 against 581).
 struct SplitPlan {
     int n_full = 0, n_tail = 0, split = 1;
     double cost = 1.0;  // of the split launch, in unit-times
@@ -1690,7 +1694,7 @@ int launch_split(const AttnArgs &a, bool neg, unsigned grid, hipStream_t st) {
 // fp32) and bf16_prescale (q rounded to bf16(c q) before the product).
 // workspace (fp32_qk, may be null): bytes for the key split of the last round;
 // too small for the planned split (empty included), the launch runs unsplit.
-// planned: a launch of few units may also run as 64-query units
+// planned: a launch of few units may also run as 64- or 128-query units
 // (attention16_short_kernel).
 int launch_attention(NineToothedStream stream, NineToothedTensor q, NineToothedTensor k, NineToothedTensor v,
                      NineToothedTensor scale, NineToothedTensor o, bool prescale, int64_t dim,

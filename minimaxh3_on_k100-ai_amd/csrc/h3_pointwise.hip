@@ -671,9 +671,9 @@ __global__ __launch_bounds__(kThreads) void rms_stream_kernel(RmsArgs a) {
 // arithmetic, so a block is one memory round trip, one reduction and its
 // stores, and the hardware's block scheduler balances the rows. Against the
 // persistent kernels, which stage the vectors in LDS first: RMSNorm + AdaLN at
-// [64, 5376] 3.6 against 10.2 us, [1000, 7168] 9.7 against 14.1 us; the gated op
-// 4.9 against 7.2 us at [256, 5376] and, with per-token rows, 48.4 against 54.9
-// us at [5726, 5376] and 86.8 against 92.8 us at [8192, 7168].
+// [64, 5376] 3.6 against 9.6 us, [1000, 7168] 9.9 against 13.9 us; the gated op
+// 4.8 against 7.2 us at [256, 5376] and, with per-token rows, 48.5 against 54.9
+// us at [5726, 5376] and 87.0 against 92.3 us at [8192, 7168].
 // A launch holds fewer than 2^32 threads along x (past them it runs only part of
 // its blocks, with no error), so it takes at most kRowBlocks rows from row0 on.
 constexpr int64_t kRowBlocks = int64_t{1} << 23;
@@ -730,7 +730,8 @@ __global__ __launch_bounds__(kThreads) void rms_row_kernel(RmsArgs a, uint32_t r
 
 // Where rms_row_kernel is the faster one (16-byte rows, 64 < W8 <= 1024), from
 // graph-timed launches of 64 to 18,000 rows of 1024 to 8192, us, row kernel
-// first:
+// first. The row counts are those of a device of 256 CUs; on a partition with
+// fewer they would scale down with them, and either kernel is right everywhere.
 //   - rows with their own modulation views (or batches past the grid's y
 //     extent): [300, 5376] 5.8 against 7.4, [8192, 7168] 76.5 against 80.4 (one
 //     row per wave);
@@ -889,9 +890,12 @@ int launch_rms_vec(const RmsArgs &a, hipStream_t stream) {
                 const int cus = stream_device_cus(stream);
                 // Three blocks per CU from 32 rows per CU on, two below, where a
                 // third one's waves get no second row to overlap with their
-                // staging: 46.1 against 48.9 us at [8192, 7168] and 74.4 against
-                // 76.8 us at [18000, 5376], but 36.6 against 34.5 us at
-                // [5726, 7168] and 29.0 against 27.7 us at [5726, 5376].
+                // staging. Three against two, us: 36.1 and 34.4 at [5726, 7168],
+                // 45.1 and 43.9 at [7200, 7168], 35.2 and 33.8 at [7200, 5376],
+                // 35.4 and 35.5 at [7700, 5376], 35.8 and 36.9 at [8192, 5376],
+                // 46.1 and 48.9 at [8192, 7168], 54.6 and 57.1 at [9500, 7168],
+                // 37.7 and 38.6 at [12000, 4096]. RMSNorm alone turns later: 25.5
+                // and 24.6 at [8192, 4096], 27.0 and 27.1 at [12000, 3072].
                 const int64_t blocks = cus > 0 ? (a.rows >= 32 * static_cast<int64_t>(cus) ? 3 : 2) * static_cast<int64_t>(cus)
                                                : kStagedBlocks;
                 const int64_t per_entry = (blocks + batch - 1) / batch;
@@ -1380,7 +1384,7 @@ __device__ __forceinline__ void head_rms(float f[8], const float w[8], float eps
 // and (b c) + (a s) -- with s' = -s in the first: negating the packed table
 // entry once (four XORs) instead of choosing a, b and the products per element
 // takes 32 of a row's VALU instructions out: q and k at 8192 tokens of 14 heads,
-// one launch each, 29.3 -> 27.8 us; the q/k/v pack 37.1 -> 36.5 us.
+// one launch each, 29.0 -> 27.7 us; the q/k/v pack 38.3 -> 37.4 us.
 __device__ __forceinline__ void rope_rotate_half(float f[8], int lane, const RopeTab &tab) {
     float partner[8];
     const int src = lane < 6 ? lane + 6 : (lane < 12 ? lane - 6 : lane);
@@ -1543,11 +1547,15 @@ __global__ __launch_bounds__(kThreads) void head_rows_loop_kernel(RopeArgs a) {
 constexpr int kHeadLoopBlocks = 4096;
 constexpr int kHeadLoopRows = 1;
 // Blocks of a persistent head-row launch: `least`, or more where they would
-// take more than `turns` batches each, up to `most`. q and k in one launch
-// (4096 to 8192 blocks, 4 turns) at 18,000 tokens of 28 heads: 94.8 us over 4096
-// blocks, 91.1 over 8192; 8192 tokens of 14 heads: 24.4 and 25.3. The pack (2048
-// to 4096 blocks, 5 turns) at 5726 tokens of 56 heads: 94.8 us over 2048, 92.6
-// over 4096; 8192 tokens of 14 heads: 37.0 and 39.9.
+// take more than `turns` batches each, up to `most`. Over `least` and over `most`
+// blocks, us: q and k in one launch (4096 and 8192 blocks, 4 turns; interleaved)
+// at 8192 tokens of 14 heads 23.4 and 24.2, 12,000 of 14 33.6 and 34.4, 8192 of
+// 28 43.1 and 42.5, 12,000 of 28 62.8 and 60.8, 18,000 of 28 93.8 and 91.3
+// (rotate-half, a launch each: 65.7 and 65.7 at 12,000 of 28, 95.6 and 92.9 at
+// 18,000). The pack (2048 and 4096, 5 turns): 2000 of 28 22.3 and 25.0, 8192 of
+// 14 36.8 and 39.7, 5726 of 28 48.9 and 50.2, 8192 of 28 68.2 and 66.7, 5726 of
+// 56 94.9 and 92.0. In between the count grows with the batches, so no size gets
+// much more than it can use.
 int64_t head_blocks(int64_t batches, int64_t least, int64_t most, int64_t turns) {
     int64_t n = batches / turns;
     n = n < least ? least : (n > most ? most : n);
