@@ -1746,7 +1746,7 @@ int launch_attention(NineToothedStream stream, NineToothedTensor q, NineToothedT
     a.Sk = static_cast<int>(kv.shape[2]);
     a.qblocks = (a.Sq + kBM - 1) / kBM;
     const int64_t grid = static_cast<int64_t>(a.B) * a.H * a.qblocks;
-    if (grid > static_cast<int64_t>(std::numeric_limits<int32_t>::max())) return kInvalid;
+    if (!launch_fits(grid, kThreadsWG)) return kInvalid;
     a.c = static_cast<float>(static_cast<float>(sc) * kLog2e);
     a.prescale = prescale;
     // Buffer loads when one head's K / V rows (plus one tile of key offsets

@@ -862,7 +862,7 @@ int launch_fp8(hipStream_t stream, const Fp8Args &a0) {
     Fp8Args a = a0;
     a.qblocks = (a.Sq + kBM - 1) / kBM;
     const int64_t grid = static_cast<int64_t>(a.B) * a.H * a.qblocks;
-    if (grid > static_cast<int64_t>(std::numeric_limits<int32_t>::max())) return kInvalid;
+    if (!launch_fits(grid, kThreadsWG)) return kInvalid;
     // Buffer loads when one head's K rows (non-overlapping) and V^T rows (each
     // at least Sk bytes apart) fit a 31-bit byte range.
     const int64_t esize = QK_FP8 ? 1 : 2, k_row = a.ks[2] * esize;
@@ -956,6 +956,7 @@ int launch_quantize(NineToothedStream stream, const NineToothedTensor &x, const 
     const int64_t rows = static_cast<int64_t>(B) * S;
     const int64_t n = rows * H * 8;  // (row, 16-dim chunk) pairs of quant_rows_kernel
     if (n >= (int64_t{1} << 31)) return kInvalid;
+    if (!d_contig && !launch_fits(static_cast<int64_t>(B) * H * ((S + 127) / 128), 256)) return kInvalid;
     if (check_only) return 0;
     hipStream_t st = as_stream(stream);
     float *amax = reinterpret_cast<float *>(dv.data);

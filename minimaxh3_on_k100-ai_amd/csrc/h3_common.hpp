@@ -133,6 +133,11 @@ inline bool rows_vec8_bytes(const View<N> &v) {
 
 inline hipStream_t as_stream(NineToothedStream s) { return static_cast<hipStream_t>(s); }
 
+// A launch holds fewer than 2^32 threads along x; given more, the runtime runs
+// part of its blocks and reports no error.
+constexpr int64_t kMaxLaunchThreads = (int64_t{1} << 32) - 1;
+inline bool launch_fits(int64_t blocks, int threads) { return blocks <= kMaxLaunchThreads / threads; }
+
 // Launch epilogue shared by all launchers: the launch status of the kernel.
 inline int launch_status() { return static_cast<int>(hipGetLastError()); }
 

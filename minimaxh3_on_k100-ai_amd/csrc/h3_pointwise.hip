@@ -674,8 +674,7 @@ __global__ __launch_bounds__(kThreads) void rms_stream_kernel(RmsArgs a) {
 // [64, 5376] 3.6 against 9.6 us, [1000, 7168] 9.9 against 13.9 us; the gated op
 // 4.8 against 7.2 us at [256, 5376] and, with per-token rows, 48.5 against 54.9
 // us at [5726, 5376] and 87.0 against 92.3 us at [8192, 7168].
-// A launch holds fewer than 2^32 threads along x (past them it runs only part of
-// its blocks, with no error), so it takes at most kRowBlocks rows from row0 on.
+// A launch takes at most kRowBlocks rows, from row0 on (launch_fits).
 constexpr int64_t kRowBlocks = int64_t{1} << 23;
 template <int VPT, int MODE>
 __global__ __launch_bounds__(kThreads) void rms_row_kernel(RmsArgs a, uint32_t row0) {
@@ -816,6 +815,7 @@ int launch_rms_vec(const RmsArgs &a, hipStream_t stream) {
         const int64_t rows_per_block4 = static_cast<int64_t>(kThreads / L) * 4;
         const bool four = (a.rows + rows_per_block4 - 1) / rows_per_block4 >= 1024;
         const int64_t per_block = four ? rows_per_block4 : kThreads / L;
+        if (!launch_fits((a.rows + per_block - 1) / per_block, kThreads)) return kInvalid;
         const unsigned grid = static_cast<unsigned>((a.rows + per_block - 1) / per_block);
         switch (L) {
 #define H3_RMS_LANES(LL)                                                                  \
@@ -916,6 +916,7 @@ int launch_rms_vec(const RmsArgs &a, hipStream_t stream) {
         }
     }
     if (!VEC && need <= 16) {
+        if (!launch_fits((a.rows + kThreads / 64 - 1) / (kThreads / 64), kThreads)) return kInvalid;
         const unsigned grid = static_cast<unsigned>((a.rows + kThreads / 64 - 1) / (kThreads / 64));
 #define H3_RMS_WAVE(GG)                                                            \
     if (need <= GG) {                                                             \
@@ -927,6 +928,7 @@ int launch_rms_vec(const RmsArgs &a, hipStream_t stream) {
 #undef H3_RMS_WAVE
     }
     const int vpt = (W8 + kThreads - 1) / kThreads;
+    if (!launch_fits(a.rows, kThreads)) return kInvalid;
     const unsigned grid = static_cast<unsigned>(a.rows);
 #define H3_RMS_BLOCK(V)                                                                \
     if (vpt <= V) {                                                                   \
@@ -1201,27 +1203,43 @@ int launch_ew(hipStream_t stream, const NineToothedTensor *in_t, const NineTooth
     const bool half = vec && Op::kUnroll == 1 && W8 % kThreads != 0 && W8 % (kThreads / 2) == 0;
     const int tb = half ? kThreads / 2 : kThreads;
     a.chunks = (W8 + tb * Op::kUnroll - 1) / (tb * Op::kUnroll);
-    const int64_t grid = a.rows * a.chunks;
-    if (grid > static_cast<int64_t>(std::numeric_limits<int32_t>::max())) return kInvalid;
-    const unsigned g = static_cast<unsigned>(grid);
-    if (index_t != nullptr) {
-        if constexpr (Op::kIndexable) {
-            if (half)
-                ew_kernel<Op, true, true, kThreads / 2><<<g, kThreads / 2, 0, stream>>>(a);
-            else if (vec)
-                ew_kernel<Op, true, true, kThreads><<<g, kThreads, 0, stream>>>(a);
+    // One launch, or pieces of whole batch entries or of one entry's rows where
+    // the rows take more blocks than a launch holds (launch_fits).
+    const int64_t max_rows = kMaxLaunchThreads / tb / a.chunks;
+    const int64_t B = out.shape[0], S = a.S, ns = S < max_rows ? S : max_rows, nb = max_rows / ns;
+    for (int64_t b0 = 0; b0 < B; b0 += nb)
+        for (int64_t s0 = 0; s0 < S; s0 += ns) {
+            EwArgs p = a;
+            p.S = S - s0 < ns ? S - s0 : ns;
+            p.rows = (B - b0 < nb ? B - b0 : nb) * p.S;
+            auto shift = [&](Rows &r) { r.p += (b0 * r.sb + s0 * r.ss) * static_cast<int64_t>(sizeof(bf16_t)); };
+            shift(p.a);
+            shift(p.c);
+            shift(p.out);
+            if (index_t == nullptr)
+                shift(p.b);
             else
-                ew_kernel<Op, false, true, kThreads><<<g, kThreads, 0, stream>>>(a);
-        } else {
-            return kInvalid;
+                p.index.p += b0 * p.index.sb + s0 * p.index.ss;
+            const unsigned g = static_cast<unsigned>(p.rows * p.chunks);
+            if (index_t != nullptr) {
+                if constexpr (Op::kIndexable) {
+                    if (half)
+                        ew_kernel<Op, true, true, kThreads / 2><<<g, kThreads / 2, 0, stream>>>(p);
+                    else if (vec)
+                        ew_kernel<Op, true, true, kThreads><<<g, kThreads, 0, stream>>>(p);
+                    else
+                        ew_kernel<Op, false, true, kThreads><<<g, kThreads, 0, stream>>>(p);
+                } else {
+                    return kInvalid;
+                }
+            } else if (half) {
+                ew_kernel<Op, true, false, kThreads / 2><<<g, kThreads / 2, 0, stream>>>(p);
+            } else if (vec) {
+                ew_kernel<Op, true, false, kThreads><<<g, kThreads, 0, stream>>>(p);
+            } else {
+                ew_kernel<Op, false, false, kThreads><<<g, kThreads, 0, stream>>>(p);
+            }
         }
-    } else if (half) {
-        ew_kernel<Op, true, false, kThreads / 2><<<g, kThreads / 2, 0, stream>>>(a);
-    } else if (vec) {
-        ew_kernel<Op, true, false, kThreads><<<g, kThreads, 0, stream>>>(a);
-    } else {
-        ew_kernel<Op, false, false, kThreads><<<g, kThreads, 0, stream>>>(a);
-    }
     return launch_status();
 }
 
@@ -1625,8 +1643,6 @@ int launch_head_rows(hipStream_t stream, const View<4> &x, const View<4> &out, c
     const bool four = (a.rows + 4 * kPerBlock - 1) / (4 * kPerBlock) >= 1024;
     const int64_t per_block = four ? 4 * kPerBlock : kPerBlock;
     const int64_t grid = (a.rows + per_block - 1) / per_block;
-    if (grid > static_cast<int64_t>(std::numeric_limits<int32_t>::max())) return kInvalid;
-    const unsigned g = static_cast<unsigned>(grid);
     if (kHeadLoopBlocks > 0 && vec && off32) {
         constexpr int64_t kBatch = kPerBlock * kHeadLoopRows;
         const int64_t needed = (a.rows + kBatch - 1) / kBatch;
@@ -1637,6 +1653,8 @@ int launch_head_rows(hipStream_t stream, const View<4> &x, const View<4> &out, c
             head_rows_loop_kernel<true, MODE, kHeadLoopRows, true><<<gl, kThreads, 0, stream>>>(a);
         return launch_status();
     }
+    if (!launch_fits(grid, kThreads)) return kInvalid;
+    const unsigned g = static_cast<unsigned>(grid);
 #define H3_HEAD_ROWS(V, R, O) \
     if (vec == V && (four ? 4 : 1) == R && off32 == O) head_rows_kernel<V, MODE, R, O><<<g, kThreads, 0, stream>>>(a);
     H3_HEAD_ROWS(true, 4, true) H3_HEAD_ROWS(true, 1, true) H3_HEAD_ROWS(true, 4, false)
@@ -2513,7 +2531,7 @@ NineToothedResult launch_h3_rope_cache(NineToothedStream stream, NineToothedTens
     const int64_t n = pos.shape[0] * 48;
     if (n == 0) return 0;
     const int64_t grid = (n + kThreads - 1) / kThreads;
-    if (grid > static_cast<int64_t>(std::numeric_limits<int32_t>::max())) return kInvalid;
+    if (!launch_fits(grid, kThreads)) return kInvalid;
     rope_cache_kernel<<<static_cast<unsigned>(grid), kThreads, 0, as_stream(stream)>>>(
         reinterpret_cast<const double *>(pos.data), pos.stride[0], pos.stride[1],
         reinterpret_cast<const float *>(pw.data), pw.stride[0], reinterpret_cast<bf16_t *>(c.data),

@@ -458,3 +458,25 @@ def test_missing_library_raises_for_every_entry_point(tmp_path):
 def test_raw_qk_norm_rope_form_is_twelve_arguments(pkg):
     raw = pkg.make_qk_norm_rope(caller="hip")
     assert raw.__code__.co_argcount == 12
+
+
+def test_launches_past_the_thread_extent_are_refused(lib):
+    """2^32 threads along x and more are past what a launch holds (the runtime
+    would run part of the blocks and report nothing): refused on the host."""
+    big = 1 << 30
+    att = t((1 << 20, 16, 1, 128))
+    code, descale = t((1 << 20, 16, 1, 128)), t((16,))
+    vcode = t((1 << 20, 16, 16, 128), (16 * 2048, 2048, 1, 16))
+    head = t((big, 1, 1, 128), (129, 129, 129, 1))  # rows the 16-byte loop does not take
+    rows, table, w = t((1, big, 512)), t((big, 64)), t((128,))
+    for name, args in [
+            ("launch_h3_full_attention", (att, att, att, scal(), att)),
+            ("launch_h3_vision_attention_72", [t((1 << 20, 16, 1, 72))] * 3 + [scal(), t((1 << 20, 16, 1, 72))]),
+            ("launch_h3_attention_planned", (att, att, att, scal(), att, t((0,)))),
+            ("launch_h3_full_attention_fp8", (code, t((1 << 20, 16, 16, 128)), vcode, descale, descale, descale, scal(),
+                                              att)),
+            ("launch_h3_rms_exact", (rows, t((512,)), scal(), rows)),
+            ("launch_h3_rms_exact", (t((1, big, 520), (0, 521, 1)), t((520,)), scal(), t((1, big, 520)))),
+            ("launch_h3_qk_norm_rope_interleaved", (head, w, scal(), table, table, head)),
+            ("launch_h3_rope_cache", (t((big, 3)), t((16,)), t((big, 48)), t((big, 48))))]:
+        assert lib.call(name, 0, *(a(lib) for a in args)) == INVALID, name

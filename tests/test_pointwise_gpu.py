@@ -585,3 +585,26 @@ def test_rms_family_special_values(pkg, oracle, device, W):
     ref_res, ref_out = oracle.gated_residual_rms_modulate_indexed(x, g_t, y, w, 1e-6, s_t, h_t, index)
     assert_bitwise(res4, ref_res, f"indexed fused residual W={W}")
     assert_bitwise(out4, ref_out, f"indexed fused modulated W={W}")
+
+
+@pytest.mark.parametrize("B,S", [(1, (1 << 24) + 3), ((1 << 13) + 1, (1 << 11) + 1)])
+def test_elementwise_rows_past_one_launch(pkg, device, B, S):
+    """More rows than one launch has blocks for (2^24 of 256 threads): parts of a
+    batch entry, or whole entries, in several launches. Against launches over
+    slices, bitwise."""
+    x, g, y = (torch.randn(B, S, 8, device=device).to(torch.bfloat16) for _ in range(3))
+    table = torch.randn(5, 8, device=device).to(torch.bfloat16)
+    index = torch.randint(0, 5, (B, S), device=device)
+    swiglu, gated, indexed = pkg.make_swiglu(), pkg.make_gated_residual(), pkg.make_gated_residual_indexed(False)
+    nan = float("nan")
+    for run in (lambda x, g, y, i, o: swiglu(x, g, o), lambda x, g, y, i, o: gated(x, g, y, o),
+                lambda x, g, y, i, o: indexed(x, table, y, i, o)):
+        out, want = torch.full_like(x, nan), torch.full_like(x, nan)
+        run(x, g, y, index, out)
+        step_b, step_s = max(1, B // 3), S if B > 1 else S // 3
+        for b in range(0, B, step_b):
+            for s in range(0, S, step_s):
+                part = (slice(b, b + step_b), slice(s, s + step_s))
+                run(x[part], g[part], y[part], index[part], want[part])
+        assert not bool(torch.isnan(want).any())
+        assert torch.equal(out, want)
